@@ -206,6 +206,12 @@ struct GemmArgs {
     // writes as an int after the partials for the reduce (0 = splits fixed
     // by the host)
     int wsplit;
+    // fp32 products on the fp32 matrix instructions (0: on the bf16 pipe by an
+    // exact three-way split of the operands, at smaller error and higher rate).
+    // k-contiguous operands only (the training forward, see model.hip).
+    int f32m;
+    // set by pt_gemm: 64 x 64 tiles (gemm_small_kernel)
+    int small;
 };
 
 // K splits of a weight gradient (A transposed, reduction over K rows) of

@@ -15,6 +15,7 @@
 // depend on scheduling (the reference accumulates with atomics).
 #include "common.h"
 
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -60,8 +61,9 @@ __device__ __forceinline__ GemmArgs gemm_shape(const GemmArgs& g0) {
 // 8 XCDs, so XCD x gets the contiguous logical range starting at
 // x*q + min(x, r) (count = 8q + r) — every XCD gets work and keeps its A rows
 // in its own L2.  Returns false for blocks beyond the count.
+template <int T = BM>
 __device__ __forceinline__ bool tile_of_range(const GemmArgs& g, int tn, int& tm_i, int& tn_i, int b) {
-    const int count = g.ntiles ? g.ntiles : ((g.M + BM - 1) / BM) * tn;
+    const int count = g.ntiles ? g.ntiles : ((g.M + T - 1) / T) * tn;
     if (b >= count) return false;
     const int q = count >> 3, r = count & 7, x = b & 7;
     const int lb = g.tile0 + x * q + min(x, r) + (b >> 3);
@@ -627,6 +629,14 @@ template <int NS> __device__ __forceinline__ void wait_stages(int later) {
     else if (NS > 2 && later == 1) wait_vm<4>();
     else wait_vm<0>();
 }
+// the same with five loads a stage, at most four stages
+__device__ __forceinline__ void wait_later5(int later) {
+    if (later >= 4) asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
+    else if (later == 3) asm volatile("s_waitcnt vmcnt(15)" ::: "memory");
+    else if (later == 2) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+    else if (later == 1) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
 // row swizzle of the [row][k] layout: conflict-free 128-bit reads of 16 rows
 // (one k group) on 32- and 64-bank LDS, and conflict-free DMA writes
 __device__ __forceinline__ int swz(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
@@ -648,6 +658,65 @@ template <bool T> __device__ __forceinline__ int dma_src(int c, int lane, int r0
     }
     const int k = 2 * c + (lane >> 5), gq = lane & 31;
     return (int)(k * ld) + r0 + 4 * (gq ^ (k & 4));
+}
+
+// The 128 x 128 tile of a wave's 2 x 2 32 x 32 accumulators out: tail
+// partials, split-K partials, and the epilogues (staged through smem where
+// they read R or apply the GELU).
+template <int EPI, bool PARTIAL>
+__device__ __forceinline__ void store_tile32(const GemmArgs& g, floatx16 (&acc32)[2][2], int tmi, int tni, int tn,
+                                             int wm, int wn, int l32, int lh, long part_stride, int bz,
+                                             float* smem) {
+    const int m0 = tmi * BM, n0 = tni * BN;
+    if (PARTIAL && g.tail_part) {
+        // tile-local partial [split][tile - tile0][BM][BN] (no bounds: the reduce masks)
+        const long t = (long)tmi * tn + tni - g.tile0;
+        float* P = g.C + ((long)bz * g.ntiles + t) * (BM * BN);
+#pragma unroll
+        for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < 2; ++tj)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    st_g4(P + (wm + 32 * ti + l32) * BN + wn + 32 * tj + 8 * q + 4 * lh,
+                          floatx4{acc32[ti][tj][4 * q], acc32[ti][tj][4 * q + 1], acc32[ti][tj][4 * q + 2],
+                                  acc32[ti][tj][4 * q + 3]});
+        return;
+    }
+    GemmArgs ge = g;
+    if (PARTIAL) ge.C = g.C + (long)bz * part_stride;   // split-K partial: a plain store
+    const uintptr_t al = PARTIAL ? (uintptr_t)ge.C | (uintptr_t)(g.ldc * 4)
+                                 : (uintptr_t)g.C | (uintptr_t)g.C2 | (uintptr_t)g.R | (uintptr_t)g.bias |
+                                       (uintptr_t)((g.ldc | g.ldc2 | g.ldr) * 4);
+    const bool vo = (al & 15) == 0;
+    if (PARTIAL || !EpiStaged<EPI>::value) {
+        // plain, bias and accumulate outputs straight from the accumulators:
+        // a store instruction covers 32 rows x 32 B, and the wave's four
+        // stores of a run (8 q + 4 lh) fill each row's 128 B segment
+        constexpr int E = PARTIAL ? EPI_STORE : EPI;
+#pragma unroll
+        for (int ti = 0; ti < 2; ++ti) {
+            const int m = m0 + wm + 32 * ti + l32;
+            if (m >= g.M) continue;
+#pragma unroll
+            for (int tj = 0; tj < 2; ++tj)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int n = n0 + wn + 32 * tj + 8 * q + 4 * lh;
+                    const floatx4 v = floatx4{acc32[ti][tj][4 * q], acc32[ti][tj][4 * q + 1],
+                                              acc32[ti][tj][4 * q + 2], acc32[ti][tj][4 * q + 3]};
+                    if (vo && n + 3 < g.N) {
+                        epi_store4<E>(ge, m, n, v);
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (n + r < g.N) epi_store<E>(ge, m, n + r, v[r]);
+                    }
+                }
+        }
+        return;
+    }
+    epilogue_staged32<EPI, false>(ge, acc32, m0, n0, wm, wn, l32, lh, smem, vo, false);
 }
 
 // One 128 x 128 tile of C (split bz of gz along K) of the logical tile
@@ -855,58 +924,507 @@ __device__ __forceinline__ void gemm_dma_tile(const GemmArgs& g0, int k_chunk0, 
     }
 
     if constexpr (W32) {
-        if (PARTIAL && g.tail_part) {
-            // tile-local partial [split][tile - tile0][BM][BN] (no bounds: the reduce masks)
-            const long t = (long)tmi * tn + tni - g.tile0;
-            float* P = g.C + ((long)bz * g.ntiles + t) * (BM * BN);
-#pragma unroll
-            for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-                for (int tj = 0; tj < 2; ++tj)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        st_g4(P + (wm + 32 * ti + l32) * BN + wn + 32 * tj + 8 * q + 4 * lh,
-                              floatx4{acc32[ti][tj][4 * q], acc32[ti][tj][4 * q + 1], acc32[ti][tj][4 * q + 2],
-                                      acc32[ti][tj][4 * q + 3]});
-            return;
-        }
-        GemmArgs ge = g;
-        if (PARTIAL) ge.C = g.C + (long)bz * part_stride;   // split-K partial: a plain store
-        const uintptr_t al = PARTIAL ? (uintptr_t)ge.C | (uintptr_t)(g.ldc * 4)
-                                     : (uintptr_t)g.C | (uintptr_t)g.C2 | (uintptr_t)g.R | (uintptr_t)g.bias |
-                                           (uintptr_t)((g.ldc | g.ldc2 | g.ldr) * 4);
-        const bool vo = (al & 15) == 0;
-        if (PARTIAL || !EpiStaged<EPI>::value) {
-            // plain, bias and accumulate outputs straight from the accumulators:
-            // a store instruction covers 32 rows x 32 B, and the wave's four
-            // stores of a run (8 q + 4 lh) fill each row's 128 B segment
-            constexpr int E = PARTIAL ? EPI_STORE : EPI;
-#pragma unroll
-            for (int ti = 0; ti < 2; ++ti) {
-                const int m = m0 + wm + 32 * ti + l32;
-                if (m >= g.M) continue;
-#pragma unroll
-                for (int tj = 0; tj < 2; ++tj)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int n = n0 + wn + 32 * tj + 8 * q + 4 * lh;
-                        const floatx4 v = floatx4{acc32[ti][tj][4 * q], acc32[ti][tj][4 * q + 1],
-                                                  acc32[ti][tj][4 * q + 2], acc32[ti][tj][4 * q + 3]};
-                        if (vo && n + 3 < g.N) {
-                            epi_store4<E>(ge, m, n, v);
-                        } else {
-#pragma unroll
-                            for (int r = 0; r < 4; ++r)
-                                if (n + r < g.N) epi_store<E>(ge, m, n + r, v[r]);
-                        }
-                    }
-            }
-            return;
-        }
-        epilogue_staged32<EPI, false>(ge, acc32, m0, n0, wm, wn, l32, lh, smem, vo, false);
+        store_tile32<EPI, PARTIAL>(g, acc32, tmi, tni, tn, wm, wn, l32, lh, part_stride, bz, smem);
         return;
     }
     gemm_epilogue<EPI, PARTIAL>(g, acc, m0, n0, wm, wn, li, lq, part_stride, smem, bz);
+}
+
+// ---------------------------------------------------------------- fp32 products on the bf16 matrix pipe
+// An fp32 value is split exactly into three bf16 terms x = h + m + l (h and m
+// round x and x - h to nearest even, l is what is left: 8 + 8 + 8 significand
+// bits and the signs of m and l cover the 24 of x).  A product keeps the six
+// terms down to 2^-18 of it (hh, hm, mh, mm, hl, lh); the three it drops are
+// below 2^-26.  A 16-k step sums its six v_mfma_f32_32x32x16_bf16, small
+// terms first, from zero and adds the result to the fp32 accumulators once,
+// where v_mfma_f32_32x32x2_f32 rounds them eight times: the relative L2 error
+// against 64 bits is 0.9e-7 / 1.7e-7 / 3.2e-7 at K = 256 / 1 024 / 4 096 where
+// the fp32 instruction's is 2.9e-7 / 5.7e-7 / 1.15e-6 (N(0, 1) operands).
+// Rates measured on this GPU with random operands: 1 738 TFLOP/s for the bf16
+// instruction (its clock drops with the operands' switching), so 290 for six,
+// against 155 for the fp32 one.
+// Denormal terms are kept by the instruction.  Inf and NaN do not survive the
+// split (inf - inf), nor do finite values past the largest bf16; they turn
+// every output of their row or column non-finite, which tile_nonfinite finds,
+// and the tile runs again on fp32 instructions.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+struct Split8 {
+    uint4 h, m, l;   // eight bf16 each
+};
+// two fp32 to bf16, round to nearest even (as an instruction: from the vector
+// conversion the compiler derives a second, single conversion per value for
+// the unpacked halves below)
+__device__ __forceinline__ unsigned pk_bf16(float a, float b) {
+    unsigned r;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+    // the mask in a vector register: v_and_b32 with a scalar or literal
+    // operand issues at half the rate (1.9 against 1.0 ns per wave measured)
+    unsigned mask;
+    asm("v_mov_b32 %0, 0xffff0000" : "=v"(mask));
+    unsigned h[4], m[4], l[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float a = x[2 * j], b = x[2 * j + 1];
+        h[j] = pk_bf16(a, b);
+        const float ra = a - __uint_as_float(h[j] << 16), rb = b - __uint_as_float(h[j] & mask);
+        m[j] = pk_bf16(ra, rb);
+        l[j] = pk_bf16(ra - __uint_as_float(m[j] << 16), rb - __uint_as_float(m[j] & mask));
+    }
+    return Split8{make_uint4(h[0], h[1], h[2], h[3]), make_uint4(m[0], m[1], m[2], m[3]),
+                  make_uint4(l[0], l[1], l[2], l[3])};
+}
+// three bf16 fragments of a row slice (each lane eight k of a row)
+struct Frag3 {
+    bf16x8 h, m, l;
+};
+__device__ __forceinline__ Frag3 split_frag(const float (&x)[8]) {
+    const Split8 s = split8(x);
+    return Frag3{__builtin_bit_cast(bf16x8, s.h), __builtin_bit_cast(bf16x8, s.m), __builtin_bit_cast(bf16x8, s.l)};
+}
+// hi[ti] += the hh term and lo[ti] += the five small terms of b x a[ti] over
+// a 16-k step for one 32-column slice
+template <int TA>
+__device__ __forceinline__ void mma_split(floatx16 (&hi)[TA], floatx16 (&lo)[TA], const Frag3 (&a)[TA],
+                                          const Frag3& b) {
+#define PT_SPLIT_TERM(acc, x, y)                      \
+    _Pragma("unroll") for (int ti = 0; ti < TA; ++ti) \
+        acc[ti] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.x, a[ti].y, acc[ti], 0, 0, 0);
+    PT_SPLIT_TERM(lo, h, m) PT_SPLIT_TERM(hi, h, h) PT_SPLIT_TERM(lo, m, h)
+    PT_SPLIT_TERM(lo, m, m) PT_SPLIT_TERM(lo, l, h) PT_SPLIT_TERM(lo, h, l)
+#undef PT_SPLIT_TERM
+}
+// whether the wave's tile holds an inf or NaN.  One in A's row reaches every
+// column of the row, one in B's column every row, so the registers of the
+// first row slice (all columns) and one register of every other slice do.
+template <int TA, int TB> __device__ __forceinline__ bool tile_nonfinite(const floatx16 (&acc)[TB][TA]) {
+    float t = 0.f;
+#pragma unroll
+    for (int tj = 0; tj < TB; ++tj)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) t = __builtin_fmaf(acc[tj][0][e], 0.f, t);
+#pragma unroll
+    for (int ti = 1; ti < TA; ++ti) t = __builtin_fmaf(acc[0][ti][0], 0.f, t);
+    return __builtin_amdgcn_ballot_w64(t != 0.f) != 0;
+}
+
+// One operand's staging slot of a thread: row r of the tile, k group kg
+// (eight k) of each 16-k stage.  T: element (k, r) at k ld + r, so a wave's
+// load covers 64 consecutive floats of a k row; else at r ld + k, two 16 B
+// loads per slot.  Loads go through a buffer resource from the tile's first
+// row (a k-contiguous operand may thus pass 2^31 bytes) and stage to the
+// operand's end, clamped below 2^31 bytes: reads past it return zero.
+template <bool T> struct SplitSlot {
+    unsigned long long base;   // address of element (0, first row of the tile)
+    int left;                  // floats from base to the operand's end
+    int vo, ld4;               // the slot's byte offset; bytes per k (T)
+    int r, kg;
+    __device__ __forceinline__ void init(const float* X, long ld, int lim, int K, int r0, int k0, int i, int tile) {
+        r = T ? i & (tile - 1) : i >> 1;
+        kg = T ? i / tile : i & 1;
+        const float* p = T ? X + (long)k0 * ld + r0 : X + (long)r0 * ld + k0;
+        const long n = T ? (long)(K - 1 - k0) * ld + lim - r0 : (long)(lim - 1 - r0) * ld + K - k0;
+        vo = T ? (int)(8 * kg * ld + r) * 4 : (int)(r * ld + 8 * kg) * 4;
+        ld4 = (int)ld * 4;
+        const unsigned long long a = (unsigned long long)p;
+        base = ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) |
+               (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a);
+        left = __builtin_amdgcn_readfirstlane((int)(n < (1L << 29) - 1 ? n : (1L << 29) - 1));
+    }
+    // the stage at k (from the first): kv k are left of the chunk.  A
+    // k-contiguous operand's row may end inside the stage (K a multiple of 4);
+    // the loads past it would read the next row and go out of range instead.
+    __device__ __forceinline__ void load(int k, int ld, int kv, float (&x)[8]) const {
+        const int o = T ? k * ld : k;
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(base + 4ull * (unsigned)o), 0, max(left - o, 0) * 4, 0x00020000);
+        if (T) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                x[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, vo + j * ld4, 0, 0));
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, 8 * kg + 4 * h < kv ? vo + 16 * h : 0x7ffffff0,
+                                                                     0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[4 * h + e] = __uint_as_float(v[e]);
+            }
+        }
+    }
+};
+
+// A 128 x 128 tile of C by 4 waves of 64 x 64.  Each operand element is read to registers once per workgroup, split there and written to
+// LDS as three bf16 planes ([row][16 k], the two 16 B halves of a row swapped
+// every eight rows: conflict-free writes and fragment reads), two stages;
+// splitting at the fragment reads instead (fp32 in LDS by DMA) splits every
+// element twice.  A stage's loads are issued one stage ahead; one barrier per
+// stage.  A transposed operand (weight gradients) is read row by row of k and
+// needs no transposition: the eight k of a slot are eight registers.
+// Same split-K, device-count, tail-partial and bias-sum rules as
+// gemm_dma_tile.
+constexpr int SPLIT_FLOATS = 2 * 2 * 3 * BM * BK / 2;   // two stages
+static_assert(SPLIT_FLOATS >= STAGE_FLOATS, "epilogue stage does not fit the operand stages");
+__device__ __forceinline__ int split_at(int r, int kg) { return r * BK + 8 * (kg ^ ((r >> 3) & 1)); }
+
+template <bool AT, bool BT, int EPI, bool PARTIAL, bool DB>
+__device__ __forceinline__ void gemm_split_tile(const GemmArgs& g0, int k_chunk0, long part_stride, int bx, int bz,
+                                                int gz, float* smem) {
+    constexpr int T = BM, TT = 2;   // tile size, 32 x 32 slices per wave side
+    constexpr int PLANE = T * BK, OPER = 3 * PLANE, STAGE = 2 * OPER;   // bf16 elements
+    const GemmArgs g = gemm_shape(g0);
+    int k_chunk = g0.Kdev ? (((g.K + gz - 1) / gz + BK - 1) / BK) * BK : k_chunk0;
+    if constexpr (PARTIAL) {
+        if (g0.Kdev && g0.wsplit) {
+            const int tiles = ((g.M + T - 1) / T) * ((g.N + T - 1) / T);
+            const int sp = pt_split_chunks(g.K, min(pt_wgrad_splits(g.K, tiles, g0.wsplit, BK), gz), BK, &k_chunk);
+            if (bx == 0 && bz == 0 && threadIdx.x == 0)
+                *reinterpret_cast<int*>(g0.C + (long)gz * (part_stride + (DB ? g0.M : 0))) = sp;
+            if (bz >= sp) return;
+        }
+    }
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tn = (g.N + T - 1) / T;
+    int tmi, tni;
+    if (!tile_of_range<T>(g, tn, tmi, tni, bx)) return;   // beyond the tile count
+    const int m0 = tmi * T, n0 = tni * T;
+    const int kbeg = bz * k_chunk;
+    const int kend = min(g.K, kbeg + k_chunk);
+    const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const int l32 = lane & 31, lh = lane >> 5;
+
+    floatx16 acc[TT][TT], low[TT][TT];   // [column slice][row slice]: the hh term, the small terms
+#pragma unroll
+    for (int j = 0; j < TT; ++j)
+#pragma unroll
+        for (int i = 0; i < TT; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[j][i][e] = low[j][i][e] = 0.f;
+
+    SplitSlot<AT> sa;
+    SplitSlot<BT> sb;
+    sa.init(g.A, g.lda, g.M, g.K, m0, kbeg, tid, T);
+    sb.init(g.B, g.ldb, g.N, g.K, n0, kbeg, tid, T);
+    __bf16* sm = reinterpret_cast<__bf16*>(smem);
+    const bool do_db = DB && AT && tni == 0;
+    float dbsum = 0.f;
+    float xa[8], xb[8];
+    auto load = [&](int it) {   // past the last stage: out of range, zeros
+        const int kv = kend - (kbeg + it * BK);
+        sa.load(it * BK, (int)g.lda, kv, xa);
+        sb.load(it * BK, (int)g.ldb, kv, xb);
+    };
+    auto put = [&](__bf16* dst, const float (&x)[8], int r, int kg) {
+        const Split8 f = split8(x);
+        __bf16* d = dst + split_at(r, kg);
+        *reinterpret_cast<uint4*>(d) = f.h;
+        *reinterpret_cast<uint4*>(d + PLANE) = f.m;
+        *reinterpret_cast<uint4*>(d + 2 * PLANE) = f.l;
+    };
+    auto stage = [&](int it) {   // the loaded stage to LDS
+        __bf16* st = sm + (it & 1) * STAGE;
+        put(st, xa, sa.r, sa.kg);
+        if (DB && AT) {   // k rows past K were loaded as zeros; summed by every tile, a branch here would
+                          // cut the loop body in two
+#pragma unroll
+            for (int j = 0; j < 8; ++j) dbsum += xa[j];
+        }
+        put(st + OPER, xb, sb.r, sb.kg);
+    };
+    auto frag = [&](const __bf16* plane, int row) {
+        const __bf16* p = plane + split_at(row, lh);
+        return Frag3{*reinterpret_cast<const bf16x8*>(p), *reinterpret_cast<const bf16x8*>(p + PLANE),
+                     *reinterpret_cast<const bf16x8*>(p + 2 * PLANE)};
+    };
+    auto mma = [&](int it) {
+        const __bf16* st = sm + (it & 1) * STAGE;
+        Frag3 a[TT];
+#pragma unroll
+        for (int t = 0; t < TT; ++t) a[t] = frag(st, wm + 32 * t + l32);
+#pragma unroll
+        for (int tj = 0; tj < TT; ++tj) mma_split(acc[tj], low[tj], a, frag(st + OPER, wn + 32 * tj + l32));
+    };
+    if (nk > 0) {
+        load(0);
+        stage(0);
+        load(1);
+        __syncthreads();
+        for (int it = 0; it + 1 < nk; ++it) {   // branch-free: the splits fill the gaps between the products
+            mma(it);
+            stage(it + 1);   // the other buffer: its readers passed the last barrier
+            load(it + 2);
+            {
+                // issue order: fragments, then products with a few of the
+                // next stage's split instructions behind each (the matrix
+                // pipe is busy 32 cycles per product), LDS writes and the
+                // loads of the stage after it last
+                __builtin_amdgcn_sched_group_barrier(0x100, 9, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+#pragma unroll
+                for (int i = 0; i < 18; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                }
+                __builtin_amdgcn_sched_group_barrier(0x200, 6, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, AT ? 16 : 4, 0);
+            }
+            __syncthreads();
+        }
+        mma(nk - 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < TT; ++j)
+#pragma unroll
+        for (int i = 0; i < TT; ++i) acc[j][i] += low[j][i];
+    {
+        __shared__ int nonfinite[NT / 64];
+        const bool nf = tile_nonfinite<TT, TT>(acc);
+        if (lane == 0) nonfinite[wave] = nf;
+        __syncthreads();
+        if (nonfinite[0] | nonfinite[1] | nonfinite[2] | nonfinite[3]) {
+            // rare: the tile again on fp32 instructions, straight from memory
+#pragma unroll
+            for (int j = 0; j < TT; ++j)
+#pragma unroll
+                for (int i = 0; i < TT; ++i)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.f;
+            for (int k0 = kbeg; k0 < kend; k0 += BK) {
+                for (int st = 0; st < 8; ++st) {
+                    const int k = k0 + 8 * lh + st;
+                    float av[TT], bv[TT];
+#pragma unroll
+                    for (int t = 0; t < TT; ++t) {
+                        const int ra = m0 + wm + 32 * t + l32, rb = n0 + wn + 32 * t + l32;
+                        av[t] = ra < g.M && k < kend ? g.A[AT ? (long)k * g.lda + ra : (long)ra * g.lda + k] : 0.f;
+                        bv[t] = rb < g.N && k < kend ? g.B[BT ? (long)k * g.ldb + rb : (long)rb * g.ldb + k] : 0.f;
+                    }
+#pragma unroll
+                    for (int tj = 0; tj < TT; ++tj)
+#pragma unroll
+                        for (int ti = 0; ti < TT; ++ti)
+                            acc[tj][ti] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[tj], av[ti], acc[tj][ti], 0, 0, 0);
+                }
+            }
+        }
+    }
+    if (DB && AT && do_db) {
+        // thread (r, kg) summed k group kg of column r; fixed-order pair sum
+        float* sh = smem;
+        sh[tid] = dbsum;
+        __syncthreads();
+        const int m = m0 + tid;
+        if (tid < T && m < g.M) {
+            const float v = sh[tid] + sh[tid + T];
+            if (PARTIAL) g.C[(long)gz * part_stride + (long)bz * g.M + m] = v;
+            else g.dbias[m] = v;
+        }
+        __syncthreads();
+    }
+    floatx16 acc32[2][2] = {{acc[0][0], acc[1][0]}, {acc[0][1], acc[1][1]}};
+    store_tile32<EPI, PARTIAL>(g, acc32, tmi, tni, tn, wm, wn, l32, lh, part_stride, bz, smem);
+}
+
+template <bool AT, bool BT, int EPI, bool PARTIAL, bool DB>
+__global__ __launch_bounds__(NT, 2) void gemm_split_kernel(const GemmArgs g0, int k_chunk0, long part_stride) {
+    __shared__ __align__(16) float smem[SPLIT_FLOATS];
+    gemm_split_tile<AT, BT, EPI, PARTIAL, DB>(g0, k_chunk0, part_stride, blockIdx.x, blockIdx.z, gridDim.z, smem);
+}
+
+// ---------------------------------------------------------------- small grids
+// A product whose 128 x 128 tiles leave CUs idle is bound by its chain of k
+// stages: one stage of a 128 x 128 tile is 0.85 us of fp32 matrix
+// instructions on each SIMD, and with two DMA stages in flight a memory
+// round trip.  Here a workgroup takes a 64 x 64 tile (four times as many
+// workgroups, each wave one 32 x 32 slice: 0.23 us of fp32 instructions or
+// six bf16 ones per stage) and keeps SM_NS - 1 = 7 stages in flight (8 KB
+// each, two workgroups per CU).  Every output still accumulates the same
+// products in the same order as in the 128 x 128 kernels, so the tile size
+// does not show in the result.  F32M: fp32 instructions, else the split (at
+// the fragment reads: a stage's operands go to LDS by DMA as they are).
+constexpr int SM_T = 64, SM_NS = 8, SM_FLOATS = SM_NS * 2 * SM_T * BK;
+// LDS layouts of a 64 x 16 operand stage as dma_at's; [k][row] swaps the
+// halves of the k rows 8..15, so the two half waves of a fragment read
+// (k = 8 lh + j) cover all banks
+template <bool T> __device__ __forceinline__ int small_at(int r, int k) {
+    return T ? k * SM_T + 4 * ((r >> 2) ^ (k & 8)) + (r & 3) : r * BK + 4 * ((k >> 2) ^ swz(r)) + (k & 3);
+}
+// wave c's 1 KB DMA chunk of a stage: 16 rows, or 4 k rows
+template <bool T> __device__ __forceinline__ int small_src(int c, int lane, int r0, long ld) {
+    if (!T) {
+        const int r = 16 * c + (lane >> 2);
+        return (int)((r0 + r) * ld) + 4 * ((lane & 3) ^ swz(r));
+    }
+    const int k = 4 * c + (lane >> 4);
+    return (int)(k * ld) + r0 + 4 * ((lane & 15) ^ (k & 8));
+}
+// wait until at most `later` stages (two loads each) are in flight
+__device__ __forceinline__ void small_wait(int later) {
+    if (later >= 6) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    else if (later == 5) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+    else if (later == 4) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else if (later == 3) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    else if (later == 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else if (later == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+template <bool AT, bool BT, int EPI, bool PARTIAL, bool DB, bool F32M>
+__device__ __forceinline__ void gemm_small_tile(const GemmArgs& g0, int k_chunk0, long part_stride, int bx, int bz,
+                                                int gz, float* smem) {
+    const GemmArgs g = gemm_shape(g0);
+    int k_chunk = g0.Kdev ? (((g.K + gz - 1) / gz + BK - 1) / BK) * BK : k_chunk0;
+    if constexpr (PARTIAL) {
+        if (g0.Kdev && g0.wsplit) {   // see gemm_dma_tile
+            const int tiles = ((g.M + SM_T - 1) / SM_T) * ((g.N + SM_T - 1) / SM_T);
+            const int sp = pt_split_chunks(g.K, min(pt_wgrad_splits(g.K, tiles, g0.wsplit, BK), gz), BK, &k_chunk);
+            if (bx == 0 && bz == 0 && threadIdx.x == 0)
+                *reinterpret_cast<int*>(g0.C + (long)gz * (part_stride + (DB ? g0.M : 0))) = sp;
+            if (bz >= sp) return;
+        }
+    }
+    constexpr int TILE = SM_T * BK;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tn = (g.N + SM_T - 1) / SM_T;
+    int tmi, tni;
+    if (!tile_of_range<SM_T>(g, tn, tmi, tni, bx)) return;   // beyond the tile count
+    const int m0 = tmi * SM_T, n0 = tni * SM_T;
+    const int kbeg = bz * k_chunk;
+    const int kend = min(g.K, kbeg + k_chunk);
+    const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int l32 = lane & 31, lh = lane >> 5;
+    // exact operand extents (host checked < 2^31 bytes)
+    const unsigned ea = (unsigned)(AT ? ((long)(g.K - 1) * g.lda + g.M) : ((long)(g.M - 1) * g.lda + g.K)) * 4u;
+    const unsigned eb = (unsigned)(BT ? ((long)(g.K - 1) * g.ldb + g.N) : ((long)(g.N - 1) * g.ldb + g.K)) * 4u;
+    const int32x4_t ra = buffer_rsrc(g.A, ea), rb = buffer_rsrc(g.B, eb);
+    const int sa = small_src<AT>(wave, lane, m0, g.lda), sb = small_src<BT>(wave, lane, n0, g.ldb);
+    const int ka = AT ? (int)g.lda : 1, kb = BT ? (int)g.ldb : 1;   // element step per k
+    auto issue = [&](int it) {
+        const int k0 = kbeg + it * BK;
+        const float* st = smem + (it % SM_NS) * 2 * TILE + wave * 256;
+        dma16(ra, st, (sa + k0 * ka) * 4);
+        dma16(rb, st + TILE, (sb + k0 * kb) * 4);
+    };
+    const bool do_db = DB && AT && tni == 0;
+    float dbsum = 0.f;
+    floatx16 hi[1][1], lo[1][1];
+    auto products = [&](auto split) {
+        constexpr bool SPLIT = decltype(split)::value;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) hi[0][0][e] = lo[0][0][e] = 0.f;
+        dbsum = 0.f;
+#pragma unroll
+        for (int t = 0; t < SM_NS - 1; ++t)
+            if (t < nk) issue(t);
+        for (int it = 0; it < nk; ++it) {
+            small_wait(min(SM_NS - 2, nk - 1 - it));
+            __syncthreads();   // every wave's loads of stage it are in LDS; stage it - 1 is consumed
+            float* Ab = smem + (it % SM_NS) * 2 * TILE;
+            float* Bb = Ab + TILE;
+            if (!(AT && BT)) {
+                // a k-contiguous operand's floats past the row end (see gemm_dma_tile)
+                const int kv = kend - (kbeg + it * BK);
+                if (kv < BK) {
+                    for (int idx = tid; idx < TILE; idx += NT) {
+                        const int r = idx / BK, k = idx % BK;
+                        if (k >= kv) {
+                            if (!AT) Ab[small_at<false>(r, k)] = 0.f;
+                            if (!BT) Bb[small_at<false>(r, k)] = 0.f;
+                        }
+                    }
+                    __syncthreads();
+                }
+            }
+            if (it + SM_NS - 1 < nk) issue(it + SM_NS - 1);
+            float a8[8], b8[8];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int k0 = 8 * lh + 4 * h;
+                if (!AT) {
+                    const float4 v = *reinterpret_cast<const float4*>(Ab + small_at<false>(wm + l32, k0));
+                    a8[4 * h] = v.x; a8[4 * h + 1] = v.y; a8[4 * h + 2] = v.z; a8[4 * h + 3] = v.w;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) a8[4 * h + e] = Ab[small_at<true>(wm + l32, k0 + e)];
+                }
+                if (!BT) {
+                    const float4 v = *reinterpret_cast<const float4*>(Bb + small_at<false>(wn + l32, k0));
+                    b8[4 * h] = v.x; b8[4 * h + 1] = v.y; b8[4 * h + 2] = v.z; b8[4 * h + 3] = v.w;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) b8[4 * h + e] = Bb[small_at<true>(wn + l32, k0 + e)];
+                }
+            }
+            if constexpr (SPLIT) {
+                const Frag3 a[1] = {split_frag(a8)};
+                mma_split(hi[0], lo[0], a, split_frag(b8));
+            } else {
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    hi[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b8[s], a8[s], hi[0][0], 0, 0, 0);
+            }
+            if (DB && AT && do_db) {   // k rows past K were loaded as zeros; columns past M are never stored
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dbsum += Ab[small_at<true>(tid & 63, 4 * wave + e)];
+            }
+        }
+    };
+    products(std::integral_constant<bool, !F32M>{});
+    if constexpr (!F32M) {
+        hi[0][0] += lo[0][0];
+        __shared__ int nonfinite[NT / 64];
+        const bool nf = tile_nonfinite<1, 1>(hi);
+        if (lane == 0) nonfinite[wave] = nf;
+        __syncthreads();
+        if (nonfinite[0] | nonfinite[1] | nonfinite[2] | nonfinite[3]) products(std::false_type{});   // rare
+    }
+    if (DB && AT && do_db) {
+        __syncthreads();
+        float* sh = smem;
+        sh[tid] = dbsum;
+        __syncthreads();
+        const int m = m0 + tid;
+        if (tid < SM_T && m < g.M) {
+            const float v = ((sh[tid] + sh[tid + 64]) + sh[tid + 128]) + sh[tid + 192];
+            if (PARTIAL) g.C[(long)gz * part_stride + (long)bz * g.M + m] = v;
+            else g.dbias[m] = v;
+        }
+    }
+    // one 32 x 32 slice per wave, straight from the accumulators
+    GemmArgs ge = g;
+    if (PARTIAL) ge.C = g.C + (long)bz * part_stride;
+    const uintptr_t al = PARTIAL ? (uintptr_t)ge.C | (uintptr_t)(g.ldc * 4)
+                                 : (uintptr_t)g.C | (uintptr_t)g.C2 | (uintptr_t)g.R | (uintptr_t)g.bias |
+                                       (uintptr_t)((g.ldc | g.ldc2 | g.ldr) * 4);
+    const bool vo = (al & 15) == 0;
+    constexpr int E = PARTIAL ? EPI_STORE : EPI;
+    const int m = m0 + wm + l32;
+    if (m < g.M) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int n = n0 + wn + 8 * q + 4 * lh;
+            const floatx4 v = floatx4{hi[0][0][4 * q], hi[0][0][4 * q + 1], hi[0][0][4 * q + 2], hi[0][0][4 * q + 3]};
+            if (vo && n + 3 < g.N) {
+                epi_store4<E>(ge, m, n, v);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (n + r < g.N) epi_store<E>(ge, m, n + r, v[r]);
+            }
+        }
+    }
+}
+
+template <bool AT, bool BT, int EPI, bool PARTIAL, bool DB, bool F32M>
+__global__ __launch_bounds__(NT) void gemm_small_kernel(const GemmArgs g0, int k_chunk0, long part_stride) {
+    __shared__ __align__(16) float smem[SM_FLOATS];
+    gemm_small_tile<AT, BT, EPI, PARTIAL, DB, F32M>(g0, k_chunk0, part_stride, blockIdx.x, blockIdx.z, gridDim.z, smem);
 }
 
 template <bool AT, bool BT, int EPI, bool PARTIAL, bool DB>
@@ -948,17 +1466,18 @@ __device__ __forceinline__ DTail dtail_plan(const GemmArgs& g, int S) {
 // them visible to every XCD, where a reduction by the last split to arrive
 // would need an agent-scope release per tail workgroup (an L2 write-back on
 // this GPU, measured slower than the unbalanced wave).
-template <bool AT, bool BT, int EPI>
+template <bool AT, bool BT, int EPI, bool SPLIT>
 __global__ __launch_bounds__(NT) void gemm_f32_dma_dtail_kernel(const GemmArgs g0, float* __restrict__ part,
                                                                int S) {
-    __shared__ __align__(16) float smem[dma_smem_floats<DMA_NS>()];
+    __shared__ __align__(16) float smem[SPLIT ? SPLIT_FLOATS : dma_smem_floats<DMA_NS>()];
     const DTail p = dtail_plan(gemm_shape(g0), S);
     const int b = blockIdx.x;
     if (b < p.full) {
         GemmArgs f = g0;
         f.tile0 = 0;
         f.ntiles = p.full;
-        gemm_dma_tile<AT, BT, EPI, false, false>(f, g0.K, 0, b, 0, 1, smem);
+        if constexpr (SPLIT) gemm_split_tile<AT, BT, EPI, false, false>(f, g0.K, 0, b, 0, 1, smem);
+        else gemm_dma_tile<AT, BT, EPI, false, false>(f, g0.K, 0, b, 0, 1, smem);
         return;
     }
     const int u = b - p.full;
@@ -968,7 +1487,8 @@ __global__ __launch_bounds__(NT) void gemm_f32_dma_dtail_kernel(const GemmArgs g
     q.tile0 = p.full;
     q.ntiles = p.R;
     q.tail_part = 1;
-    gemm_dma_tile<AT, BT, EPI, true, false>(q, p.kc, 0, u % p.R, u / p.R, p.s2, smem);
+    if constexpr (SPLIT) gemm_split_tile<AT, BT, EPI, true, false>(q, p.kc, 0, u % p.R, u / p.R, p.s2, smem);
+    else gemm_dma_tile<AT, BT, EPI, true, false>(q, p.kc, 0, u % p.R, u / p.R, p.s2, smem);
 }
 
 // The tail tiles of gemm_f32_dma_dtail_kernel: 16 workgroups per tail tile
@@ -1007,112 +1527,14 @@ __global__ __launch_bounds__(256) void dtail_reduce_kernel(const GemmArgs g0, co
 }
 
 // ---------------------------------------------------------------- residual + LayerNorm
-// C = A W^T + bias + R (a pre-LN block's residual add, EPI_BIAS_RESID) at
-// N = 256, followed in the same launch by the LayerNorm of C's rows that the
-// next stage reads: Y = LN(C) lnw + lnb with its mean and rstd.  The unfused
-// pair is the DMA kernel's EPI_BIAS_RESID then ln_fwd_kernel, which reads C
-// back from HBM.  A workgroup owns BMR (64 or 32) full rows: a BMR x 256
-// tile, the four waves side by side, each a BMR x 64 sub-tile of
-// v_mfma_f32_32x32x2_f32 tiles (2 x 2 or 1 x 2) with the DMA kernel's operand
-// order, so every output accumulates the same products in the same order.  Per 16-k stage
-// the A rows (one 16-row chunk) and W rows (four chunks) go global -> LDS by
-// DMA, two stages deep.  The tile leaves through LDS in 32-row halves; a
-// wave then takes eight rows, one float4 per lane, adds bias and residual in
-// epi_store4_r's order and normalises in ln_fwd_kernel's order (two-pass
-// mean / variance by wave sums, eps 1e-5), so C, Y, mean and rstd equal the
-// unfused pair's bit for bit.  K % 16 == 0, N = 256 (host checked).
-// BF: A and W hold bf16 (the mixed-precision variant's activations and weight
-// copies; K, lda, ldb in float units, 2 bf16 per float) and the products run
-// on v_mfma_f32_32x32x16_bf16 in gemm_bs32_kernel's fragment order; YB: Y is
-// stored in bf16 (round to nearest even), ldy in bf16 elements.
 constexpr int RL_BM = 64, RL_N = 256, RL_SST = RL_N + 4;
-template <bool BF, bool YB, int BMR = RL_BM>
-__global__ __launch_bounds__(NT) void gemm_resid_ln_kernel(const GemmArgs g0, const float* __restrict__ lnw,
-        const float* __restrict__ lnb, float* __restrict__ Y, long ldy, float* __restrict__ mean,
-        float* __restrict__ rstd) {
-    const GemmArgs g = gemm_shape(g0);
-    static_assert(BMR == 128 || BMR == 64 || BMR == 32, "128-, 64- or 32-row tiles");
-    static_assert(BF || BMR <= 64, "fp32 operands: 64- or 32-row tiles");
-    constexpr int TM = BMR / 32;   // 32-row MFMA tiles per wave
-    const int m0 = blockIdx.x * BMR;
-    if (m0 >= g.M) return;   // beyond the (device) row count
-    constexpr int TA = BMR * BK, TB = RL_N * BK, STAGE = TA + TB;
-    constexpr int SMEM = 2 * STAGE > 32 * RL_SST ? 2 * STAGE : 32 * RL_SST;
-    __shared__ __align__(16) float smem[SMEM];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l32 = lane & 31, lh = lane >> 5;
-    const int wn = 64 * wave;
-    floatx16 acc[TM][2];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    // exact operand extents (host checked < 2^31 bytes): rows past M read zeros
-    const unsigned ea = (unsigned)(((long)(g.M - 1) * g.lda + g.K) * 4);
-    const unsigned eb = (unsigned)(((long)(RL_N - 1) * g.ldb + g.K) * 4);
-    const int32x4_t ra = buffer_rsrc(g.A, ea), rb = buffer_rsrc(g.B, eb);
-    // A's 16-row chunks: chunk wave (and wave + 4 for 128-row tiles)
-    const int sa = dma_src<false>(wave, lane, m0, g.lda), sa2 = dma_src<false>(wave + 4, lane, m0, g.lda);
-    int sb[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) sb[j] = dma_src<false>(4 * wave + j, lane, 0, g.ldb);
-    auto issue = [&](int tile) {
-        const int k0 = tile * BK;
-        const float* st = smem + (tile & 1) * STAGE;
-        if (wave < BMR / 16) dma16(ra, st + wave * 256, (sa + k0) * 4);
-        if (BMR == 128) dma16(ra, st + (wave + 4) * 256, (sa2 + k0) * 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) dma16(rb, st + TA + (4 * wave + j) * 256, (sb[j] + k0) * 4);
-    };
-    const int nk = g.K / BK;
-    issue(0);
-    for (int it = 0; it < nk; ++it) {
-        wait_vm<0>();      // this wave's loads of tile it have landed
-        __syncthreads();   // every wave's have; tile it - 1 is consumed
-        if (it + 1 < nk) issue(it + 1);
-        const float* Ab = smem + (it & 1) * STAGE;
-        const float* Bb = Ab + TA;
-        if constexpr (BF) {
-#pragma unroll
-            for (int st = 0; st < 2; ++st) {
-                bf16x8 ah[TM], bh[2];
-#pragma unroll
-                for (int t = 0; t < TM; ++t)
-                    ah[t] = *reinterpret_cast<const bf16x8*>(Ab + dma_at<false>(32 * t + l32, 4 * (2 * st + lh)));
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-                    bh[t] = *reinterpret_cast<const bf16x8*>(Bb + dma_at<false>(wn + 32 * t + l32, 4 * (2 * st + lh)));
-#pragma unroll
-                for (int ti = 0; ti < TM; ++ti)
-#pragma unroll
-                    for (int tj = 0; tj < 2; ++tj)
-                        acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh[tj], ah[ti], acc[ti][tj], 0, 0, 0);
-            }
-            continue;
-        }
-        float a8[TM][8], b8[2][8];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int k0 = 8 * lh + 4 * h;
-                if (t < TM) {
-                    const float4 va = *reinterpret_cast<const float4*>(Ab + dma_at<false>(32 * t + l32, k0));
-                    a8[t][4 * h] = va.x; a8[t][4 * h + 1] = va.y; a8[t][4 * h + 2] = va.z; a8[t][4 * h + 3] = va.w;
-                }
-                const float4 vb = *reinterpret_cast<const float4*>(Bb + dma_at<false>(wn + 32 * t + l32, k0));
-                b8[t][4 * h] = vb.x; b8[t][4 * h + 1] = vb.y; b8[t][4 * h + 2] = vb.z; b8[t][4 * h + 3] = vb.w;
-            }
-#pragma unroll
-        for (int st = 0; st < 8; ++st)
-#pragma unroll
-            for (int ti = 0; ti < TM; ++ti)
-#pragma unroll
-                for (int tj = 0; tj < 2; ++tj)
-                    acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x2f32(b8[tj][st], a8[ti][st], acc[ti][tj], 0, 0, 0);
-    }
+// The residual product's epilogue: bias + residual, C, then the LayerNorm of
+// each row (see gemm_resid_ln_kernel); smem: 32 x RL_SST floats.
+template <bool YB, int TM>
+__device__ __forceinline__ void resid_ln_epilogue(const GemmArgs& g, const floatx16 (&acc)[TM][2], int m0, int wave,
+        int lane, const float* __restrict__ lnw, const float* __restrict__ lnb, float* __restrict__ Y, long ldy,
+        float* __restrict__ mean, float* __restrict__ rstd, float* smem) {
+    const int l32 = lane & 31, lh = lane >> 5, wn = 64 * wave;
     // register r of lane (l32, lh) of acc[ti][tj] holds
     // C[32 ti + l32][wn + 32 tj + 8 (r / 4) + 4 lh + r % 4]; half h = rows 32 h ..
     const floatx4 bv = ld_v4(g.bias + 4 * lane);
@@ -1163,6 +1585,274 @@ __global__ __launch_bounds__(NT) void gemm_resid_ln_kernel(const GemmArgs g0, co
                 *reinterpret_cast<float4*>(Y + (long)m * ldy + 4 * lane) = o;
         }
     }
+}
+
+// C = A W^T + bias + R (a pre-LN block's residual add, EPI_BIAS_RESID) at
+// N = 256, followed in the same launch by the LayerNorm of C's rows that the
+// next stage reads: Y = LN(C) lnw + lnb with its mean and rstd.  The unfused
+// pair is the DMA kernel's EPI_BIAS_RESID then ln_fwd_kernel, which reads C
+// back from HBM.  A workgroup owns BMR (64 or 32) full rows: a BMR x 256
+// tile, the four waves side by side, each a BMR x 64 sub-tile of
+// v_mfma_f32_32x32x2_f32 tiles (2 x 2 or 1 x 2) with the DMA kernel's operand
+// order, so every output accumulates the same products in the same order.  Per 16-k stage
+// the A rows (one 16-row chunk) and W rows (four chunks) go global -> LDS by
+// DMA, two stages deep.  The tile leaves through LDS in 32-row halves; a
+// wave then takes eight rows, one float4 per lane, adds bias and residual in
+// epi_store4_r's order and normalises in ln_fwd_kernel's order (two-pass
+// mean / variance by wave sums, eps 1e-5), so C, Y, mean and rstd equal the
+// unfused pair's bit for bit.  K % 16 == 0, N = 256 (host checked).
+// BF: A and W hold bf16 (the mixed-precision variant's activations and weight
+// copies; K, lda, ldb in float units, 2 bf16 per float) and the products run
+// on v_mfma_f32_32x32x16_bf16 in gemm_bs32_kernel's fragment order; YB: Y is
+// stored in bf16 (round to nearest even), ldy in bf16 elements.
+template <bool BF, bool YB, int BMR = RL_BM, int NS = 2, bool SPL = false>
+__global__ __launch_bounds__(NT) void gemm_resid_ln_kernel(const GemmArgs g0, const float* __restrict__ lnw,
+        const float* __restrict__ lnb, float* __restrict__ Y, long ldy, float* __restrict__ mean,
+        float* __restrict__ rstd) {
+    const GemmArgs g = gemm_shape(g0);
+    static_assert(BMR == 128 || BMR == 64 || BMR == 32, "128-, 64- or 32-row tiles");
+    static_assert(BF || BMR <= 64, "fp32 operands: 64- or 32-row tiles");
+    constexpr int TM = BMR / 32;   // 32-row MFMA tiles per wave
+    const int m0 = blockIdx.x * BMR;
+    if (m0 >= g.M) return;   // beyond the (device) row count
+    constexpr int TA = BMR * BK, TB = RL_N * BK, STAGE = TA + TB;
+    constexpr int SMEM = NS * STAGE > 32 * RL_SST ? NS * STAGE : 32 * RL_SST;
+    __shared__ __align__(16) float smem[SMEM];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l32 = lane & 31, lh = lane >> 5;
+    const int wn = 64 * wave;
+    floatx16 acc[TM][2];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    // exact operand extents (host checked < 2^31 bytes): rows past M read zeros
+    const unsigned ea = (unsigned)(((long)(g.M - 1) * g.lda + g.K) * 4);
+    const unsigned eb = (unsigned)(((long)(RL_N - 1) * g.ldb + g.K) * 4);
+    const int32x4_t ra = buffer_rsrc(g.A, ea), rb = buffer_rsrc(g.B, eb);
+    // A's 16-row chunks: chunk wave (and wave + 4 for 128-row tiles)
+    const int sa = dma_src<false>(wave, lane, m0, g.lda), sa2 = dma_src<false>(wave + 4, lane, m0, g.lda);
+    int sb[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sb[j] = dma_src<false>(4 * wave + j, lane, 0, g.ldb);
+    auto issue = [&](int tile) {
+        const int k0 = tile * BK;
+        const float* st = smem + (tile % NS) * STAGE;
+        if (wave < BMR / 16) dma16(ra, st + wave * 256, (sa + k0) * 4);
+        if (BMR == 128) dma16(ra, st + (wave + 4) * 256, (sa2 + k0) * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dma16(rb, st + TA + (4 * wave + j) * 256, (sb[j] + k0) * 4);
+    };
+    const int nk = g.K / BK;
+    floatx16 low[SPL ? TM : 1][2];
+    auto products = [&](auto split) {
+        constexpr bool SPLIT = decltype(split)::value;
+#pragma unroll
+        for (int t = 0; t < NS - 1; ++t)
+            if (t < nk) issue(t);
+        for (int it = 0; it < nk; ++it) {
+            // this wave's loads of tile it have landed (the first BMR / 16
+            // waves have five a stage in flight, the others four)
+            if constexpr (NS == 2) wait_vm<0>();
+            else if (wave < BMR / 16) wait_later5(min(NS - 2, nk - 1 - it));
+            else wait_stages<NS>(min(NS - 2, nk - 1 - it));
+            __syncthreads();   // every wave's have; tile it - 1 is consumed
+            if (it + NS - 1 < nk) issue(it + NS - 1);
+            const float* Ab = smem + (it % NS) * STAGE;
+            const float* Bb = Ab + TA;
+            if constexpr (BF) {
+#pragma unroll
+                for (int st = 0; st < 2; ++st) {
+                    bf16x8 ah[TM], bh[2];
+#pragma unroll
+                    for (int t = 0; t < TM; ++t)
+                        ah[t] = *reinterpret_cast<const bf16x8*>(Ab + dma_at<false>(32 * t + l32, 4 * (2 * st + lh)));
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        bh[t] = *reinterpret_cast<const bf16x8*>(Bb + dma_at<false>(wn + 32 * t + l32, 4 * (2 * st + lh)));
+#pragma unroll
+                    for (int ti = 0; ti < TM; ++ti)
+#pragma unroll
+                        for (int tj = 0; tj < 2; ++tj)
+                            acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bh[tj], ah[ti], acc[ti][tj], 0, 0, 0);
+                }
+                continue;
+            }
+            float a8[TM][8], b8[2][8];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int k0 = 8 * lh + 4 * h;
+                    if (t < TM) {
+                        const float4 va = *reinterpret_cast<const float4*>(Ab + dma_at<false>(32 * t + l32, k0));
+                        a8[t][4 * h] = va.x; a8[t][4 * h + 1] = va.y; a8[t][4 * h + 2] = va.z; a8[t][4 * h + 3] = va.w;
+                    }
+                    const float4 vb = *reinterpret_cast<const float4*>(Bb + dma_at<false>(wn + 32 * t + l32, k0));
+                    b8[t][4 * h] = vb.x; b8[t][4 * h + 1] = vb.y; b8[t][4 * h + 2] = vb.z; b8[t][4 * h + 3] = vb.w;
+                }
+            if constexpr (SPLIT) {
+                static_assert(!SPLIT || TM == 1, "split at the reads: 32-row tiles");
+                const Frag3 a[1] = {split_frag(a8[0])};
+#pragma unroll
+                for (int tj = 0; tj < 2; ++tj) {
+                    floatx16 (&h1)[1] = *reinterpret_cast<floatx16 (*)[1]>(&acc[0][tj]);
+                    floatx16 (&l1)[1] = *reinterpret_cast<floatx16 (*)[1]>(&low[0][tj]);
+                    mma_split(h1, l1, a, split_frag(b8[tj]));
+                }
+            } else {
+#pragma unroll
+                for (int st = 0; st < 8; ++st)
+#pragma unroll
+                    for (int ti = 0; ti < TM; ++ti)
+#pragma unroll
+                        for (int tj = 0; tj < 2; ++tj)
+                            acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x2f32(b8[tj][st], a8[ti][st], acc[ti][tj], 0, 0, 0);
+            }
+        }
+    };
+    if constexpr (SPL) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) low[0][j][e] = 0.f;
+    }
+    products(std::integral_constant<bool, SPL>{});
+    if constexpr (SPL) {
+        acc[0][0] += low[0][0];
+        acc[0][1] += low[0][1];
+        __shared__ int nonfinite[NT / 64];
+        const floatx16 cols[2][1] = {{acc[0][0]}, {acc[0][1]}};
+        const bool nf = tile_nonfinite<1, 2>(cols);
+        if (lane == 0) nonfinite[wave] = nf;
+        __syncthreads();
+        if (nonfinite[0] | nonfinite[1] | nonfinite[2] | nonfinite[3]) {   // rare: the tile again in fp32
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[0][j][e] = 0.f;
+            products(std::false_type{});
+        }
+    }
+    resid_ln_epilogue<YB, TM>(g, acc, m0, wave, lane, lnw, lnb, Y, ldy, mean, rstd, smem);
+}
+
+// gemm_resid_ln_kernel for fp32 operands on the bf16 pipe: 64 x 256 tiles, the
+// operands split while staged as in gemm_split_tile (two W slots per thread,
+// the A slots on the first waves) and its products in its order, so C equals
+// the unfused product's bit for bit.
+template <bool YB>
+__global__ __launch_bounds__(NT, 2) void gemm_split_resid_ln_kernel(const GemmArgs g0, const float* __restrict__ lnw,
+        const float* __restrict__ lnb, float* __restrict__ Y, long ldy, float* __restrict__ mean,
+        float* __restrict__ rstd) {
+    const GemmArgs g = gemm_shape(g0);
+    constexpr int R = 64, TM = R / 32, PA = R * BK, PB = RL_N * BK, STAGE = 3 * (PA + PB);   // bf16 elements
+    const int m0 = blockIdx.x * R;
+    if (m0 >= g.M) return;   // beyond the (device) row count
+    __shared__ __align__(16) float smem[STAGE];   // two stages
+    static_assert(STAGE >= 32 * RL_SST, "epilogue stage does not fit the operand stages");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l32 = lane & 31, lh = lane >> 5, wn = 64 * wave;
+    __bf16* sm = reinterpret_cast<__bf16*>(smem);
+    SplitSlot<false> sa, sb0, sb1;
+    sa.init(g.A, g.lda, g.M, g.K, m0, 0, tid & (2 * R - 1), R);
+    const bool does_a = tid < 2 * R;
+    sb0.init(g.B, g.ldb, RL_N, g.K, 0, 0, tid, RL_N);
+    sb1.init(g.B, g.ldb, RL_N, g.K, 0, 0, tid + NT, RL_N);
+    float xa[8], x0[8], x1[8];
+    const int nk = g.K / BK;
+    auto load = [&](int it) {
+        const int kv = g.K - it * BK;
+        if (does_a) sa.load(it * BK, (int)g.lda, kv, xa);
+        sb0.load(it * BK, (int)g.ldb, kv, x0);
+        sb1.load(it * BK, (int)g.ldb, kv, x1);
+    };
+    auto put = [&](__bf16* dst, int plane, const float (&x)[8], int r, int kg) {
+        const Split8 f = split8(x);
+        __bf16* d = dst + split_at(r, kg);
+        *reinterpret_cast<uint4*>(d) = f.h;
+        *reinterpret_cast<uint4*>(d + plane) = f.m;
+        *reinterpret_cast<uint4*>(d + 2 * plane) = f.l;
+    };
+    auto stage = [&](int it) {
+        __bf16* st = sm + (it & 1) * STAGE;
+        if (does_a) put(st, PA, xa, sa.r, sa.kg);
+        put(st + 3 * PA, PB, x0, sb0.r, sb0.kg);
+        put(st + 3 * PA, PB, x1, sb1.r, sb1.kg);
+    };
+    floatx16 hi[2][TM], lo[2][TM];   // [column slice][row slice]
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) hi[j][i][e] = lo[j][i][e] = 0.f;
+    auto frag = [&](const __bf16* p, int plane) {
+        return Frag3{*reinterpret_cast<const bf16x8*>(p), *reinterpret_cast<const bf16x8*>(p + plane),
+                     *reinterpret_cast<const bf16x8*>(p + 2 * plane)};
+    };
+    auto mma = [&](int it) {
+        const __bf16* st = sm + (it & 1) * STAGE;
+        Frag3 a[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) a[i] = frag(st + split_at(32 * i + l32, lh), PA);
+#pragma unroll
+        for (int tj = 0; tj < 2; ++tj)
+            mma_split(hi[tj], lo[tj], a, frag(st + 3 * PA + split_at(wn + 32 * tj + l32, lh), PB));
+    };
+    load(0);
+    stage(0);
+    load(1);
+    __syncthreads();
+    for (int it = 0; it + 1 < nk; ++it) {
+        mma(it);
+        stage(it + 1);
+        load(it + 2);
+        __syncthreads();
+    }
+    mma(nk - 1);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) hi[j][i] += lo[j][i];
+    {
+        __shared__ int nonfinite[NT / 64];
+        const bool nf = tile_nonfinite<TM, 2>(hi);
+        if (lane == 0) nonfinite[wave] = nf;
+        __syncthreads();
+        if (nonfinite[0] | nonfinite[1] | nonfinite[2] | nonfinite[3]) {
+            // rare: the tile again on fp32 instructions, straight from memory
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) hi[j][i][e] = 0.f;
+            for (int k0 = 0; k0 < g.K; k0 += BK)
+                for (int st = 0; st < 8; ++st) {
+                    const int k = k0 + 8 * lh + st;
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) {
+                        const int ra = m0 + 32 * i + l32;
+                        const float av = ra < g.M ? g.A[(long)ra * g.lda + k] : 0.f;
+#pragma unroll
+                        for (int tj = 0; tj < 2; ++tj)
+                            hi[tj][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                g.B[(long)(wn + 32 * tj + l32) * g.ldb + k], av, hi[tj][i], 0, 0, 0);
+                    }
+                }
+        }
+    }
+    floatx16 acc[TM][2];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        acc[i][0] = hi[0][i];
+        acc[i][1] = hi[1][i];
+    }
+    resid_ln_epilogue<YB, TM>(g, acc, m0, wave, lane, lnw, lnb, Y, ldy, mean, rstd, smem);
 }
 
 // The LayerNorm backward fused into the bf16 dX product that feeds it (the
@@ -1319,12 +2009,12 @@ __global__ __launch_bounds__(NT) void gemm_dx_lnbwd_kernel(const GemmArgs g0, co
 template <bool AT, bool BT, int EPI, bool PARTIAL>
 __global__ __launch_bounds__(NT) void gemm_f32_dma_grouped_kernel(const GroupedGemm* __restrict__ gs,
                                                                   const int* __restrict__ item_group) {
-    __shared__ __align__(16) float smem[dma_smem_floats<DMA_NS>()];
+    __shared__ __align__(16) float smem[SPLIT_FLOATS];
     const int gi = __builtin_amdgcn_readfirstlane(item_group[blockIdx.x]);
     const int local = (int)blockIdx.x - gs[gi].first;
     const int tiles = gs[gi].tiles;
-    gemm_dma_tile<AT, BT, EPI, PARTIAL, false>(gs[gi].g, gs[gi].k_chunk, gs[gi].part_stride, local % tiles,
-                                               local / tiles, gs[gi].splits, smem);
+    gemm_split_tile<AT, BT, EPI, PARTIAL, false>(gs[gi].g, gs[gi].k_chunk, gs[gi].part_stride, local % tiles,
+                                                     local / tiles, gs[gi].splits, smem);
 }
 
 // Fixed-order sums of grouped split-K partials: chunk c covers 1024
@@ -2157,10 +2847,22 @@ double launch_flops(const GemmArgs& g) {
 template <bool AT, bool BT, int EPI, bool PARTIAL, bool DB, bool VEC>
 void launch(const GemmArgs& g, dim3 grid, int k_chunk, long part_stride, hipStream_t s) {
     const int slot = pt_prof_open(s);
-    if (VEC && g.dma)
-        hipLaunchKernelGGL((gemm_f32_dma_kernel<AT, BT, EPI, PARTIAL, DB>), grid, dim3(NT), 0, s, g, k_chunk,
+    if (VEC && g.dma && g.small) {
+        if (!g.f32m)
+            hipLaunchKernelGGL((gemm_small_kernel<AT, BT, EPI, PARTIAL, DB, false>), grid, dim3(NT), 0, s, g, k_chunk,
+                               part_stride);
+        else if constexpr (!AT && !BT)
+            hipLaunchKernelGGL((gemm_small_kernel<AT, BT, EPI, PARTIAL, DB, true>), grid, dim3(NT), 0, s, g, k_chunk,
+                               part_stride);
+    } else if (VEC && g.dma && !g.f32m) {
+        hipLaunchKernelGGL((gemm_split_kernel<AT, BT, EPI, PARTIAL, DB>), grid, dim3(NT), 0, s, g, k_chunk,
                            part_stride);
-    else
+    } else if (VEC && g.dma) {
+        // the training forward's layouts
+        if constexpr (!AT && !BT)
+            hipLaunchKernelGGL((gemm_f32_dma_kernel<AT, BT, EPI, PARTIAL, DB>), grid, dim3(NT), 0, s, g, k_chunk,
+                               part_stride);
+    } else
         hipLaunchKernelGGL((gemm_f32_kernel<AT, BT, EPI, PARTIAL, DB, VEC>), grid, dim3(NT), 0, s, g, k_chunk,
                            part_stride);
     pt_prof_close(slot, g_gemm_class, launch_flops(g), s);
@@ -2358,6 +3060,18 @@ static bool dma_ok(const GemmArgs& g) {
            dma_fits(g.b_t ? g.K : g.N, g.b_t ? g.N : g.K, g.ldb);
 }
 
+// The split kernels rebase a k-contiguous operand at each tile's first row
+// (so only a tile's rows count) and a transposed one at the chunk's first k:
+// their offsets must stay below 2^31 bytes (2^29 floats, half of it for the
+// clamped extent)
+static bool split_fits(int rows, int cols, long ld, bool t) {
+    return t ? dma_fits(rows, cols, ld) : 2L * BM * ld + cols < (1L << 28);
+}
+static bool split_ok(const GemmArgs& g) {
+    return split_fits(g.a_t ? g.K : g.M, g.a_t ? g.M : g.K, g.lda, g.a_t) &&
+           split_fits(g.b_t ? g.K : g.N, g.b_t ? g.N : g.K, g.ldb, g.b_t);
+}
+
 // ---- bf16 storage (GemmArgs::bs)
 // two DMA stages: measured faster than three or four at the trunk shapes
 // (149 504 x {256, 768, 1024} x {256, 1024}): the smaller LDS footprint
@@ -2534,7 +3248,7 @@ bool pt_gemm_resid_ln_fits(const GemmArgs& g) {
                          (uintptr_t)((g.lda | g.ldb) * (g.bs ? 2 : 4));
     const bool prec_ok = g.bs ? (g.K % 32 == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0) : (g.prec == 0 && g.K % BK == 0);
     return g.N == RL_N && g.M > 0 && prec_ok && !g.a_t && !g.b_t && g.epi == EPI_BIAS_RESID && !g.obf && g.bias &&
-           g.R && (al & 15) == 0 && !g.Kdev && dma_ok(resid_ln_float_units(g));
+           g.R && (al & 15) == 0 && !g.Kdev && (g.bs || g.f32m ? dma_ok(resid_ln_float_units(g)) : split_ok(g));
 }
 int pt_gemm_resid_ln(const GemmArgs& g, const float* lnw, const float* lnb, float* y, long ldy, float* mean,
                      float* rstd, hipStream_t s, int ybf) {
@@ -2560,8 +3274,25 @@ int pt_gemm_resid_ln(const GemmArgs& g, const float* lnw, const float* lnb, floa
         else hipLaunchKernelGGL((gemm_resid_ln_kernel<true, false, 128>), grid, blk, 0, s, f, lnw, lnb, y, ldy, mean, rstd);
     } else {
         const dim3 grid(pt_cdiv(g.M, 32));
-        if (ybf) hipLaunchKernelGGL((gemm_resid_ln_kernel<false, true, 32>), grid, blk, 0, s, f, lnw, lnb, y, ldy, mean, rstd);
-        else hipLaunchKernelGGL((gemm_resid_ln_kernel<false, false, 32>), grid, blk, 0, s, f, lnw, lnb, y, ldy, mean, rstd);
+        // up to one 32-row tile per CU: six stages in flight (110 KB of LDS),
+        // a lone tile is bound by its chain of stages
+        const bool deep = (int)grid.x <= pt_cu_count();
+#define PT_RLN(kernel, gr)                                                                                     \
+    if (ybf) hipLaunchKernelGGL((kernel(true)), gr, blk, 0, s, f, lnw, lnb, y, ldy, mean, rstd);               \
+    else hipLaunchKernelGGL((kernel(false)), gr, blk, 0, s, f, lnw, lnb, y, ldy, mean, rstd)
+#define PT_RLN_F32(yb) gemm_resid_ln_kernel<false, yb, 32>
+#define PT_RLN_F32_DEEP(yb) gemm_resid_ln_kernel<false, yb, 32, 6>
+#define PT_RLN_SPLIT_DEEP(yb) gemm_resid_ln_kernel<false, yb, 32, 6, true>
+#define PT_RLN_SPLIT(yb) gemm_split_resid_ln_kernel<yb>
+        if (g.f32m && deep) { PT_RLN(PT_RLN_F32_DEEP, grid); }
+        else if (g.f32m) { PT_RLN(PT_RLN_F32, grid); }
+        else if (deep) { PT_RLN(PT_RLN_SPLIT_DEEP, grid); }
+        else { PT_RLN(PT_RLN_SPLIT, dim3(pt_cdiv(g.M, 64))); }
+#undef PT_RLN
+#undef PT_RLN_F32
+#undef PT_RLN_F32_DEEP
+#undef PT_RLN_SPLIT_DEEP
+#undef PT_RLN_SPLIT
     }
     PT_LAUNCH_CHECK();
     pt_prof_close(slot, g_gemm_class, 2.0 * g.M * (double)g.N * g.K, s);
@@ -2602,7 +3333,10 @@ int pt_dx_lnbwd(const GemmArgs& g, const float* x, const float* w, const float* 
 template <bool AT, bool BT, int EPI>
 static void launch_dtail(const GemmArgs& g, int tiles, int S, float* ws, hipStream_t s) {
     const int slot = pt_prof_open(s);
-    hipLaunchKernelGGL((gemm_f32_dma_dtail_kernel<AT, BT, EPI>), dim3(tiles + S), dim3(NT), 0, s, g, ws, S);
+    if (g.f32m)
+        hipLaunchKernelGGL((gemm_f32_dma_dtail_kernel<AT, BT, EPI, false>), dim3(tiles + S), dim3(NT), 0, s, g, ws, S);
+    else
+        hipLaunchKernelGGL((gemm_f32_dma_dtail_kernel<AT, BT, EPI, true>), dim3(tiles + S), dim3(NT), 0, s, g, ws, S);
     pt_prof_close(slot, g_gemm_class, launch_flops(g), s);
     hipLaunchKernelGGL(dtail_reduce_kernel<EPI>, dim3(S * DTAIL_RED_WG), dim3(256), 0, s, g, (const float*)ws, S);
 }
@@ -2637,7 +3371,8 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
                      ((uintptr_t)g.B & 15) == 0;
     // bf16 products need the 128-bit operand path; other shapes stay fp32
     const bool bf = g.prec == 1 && vec;
-    g.dma = vec && dma_ok(g);
+    PT_REQUIRE(!g.f32m || (!g.a_t && !g.b_t), "gemm: fp32 instructions need k-contiguous operands");
+    g.dma = vec && (bf || g.f32m ? dma_ok(g) : split_ok(g));
     const int bk = bf && !g.dma ? BK2 : BK;
     const int tm = pt_cdiv(g.M, BM), tn = pt_cdiv(g.N, BN);
     const int tiles = tm * tn;
@@ -2667,6 +3402,7 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
     // 256 x 256 weight gradient at 37.4k of 49.7k rows: 150 us with 500
     // workgroups of which 256 worked, 61 us with the 256 alone)
     const bool wsplit_ok = g.a_t && g.Kdev && !bf && vec && g.dma && (g.epi == EPI_STORE || g.epi == EPI_ACCUM);
+    const int tiles_s = pt_cdiv(g.M, SM_T) * pt_cdiv(g.N, SM_T);
     int splits = 1;
     if (g.a_t) {
         splits = pt_wgrad_splits(g.K, tiles, cu, bk, wsplit_ok);
@@ -2678,6 +3414,35 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
         if (splits < 1) splits = 1;
     }
     if (g.Mdev) splits = 1;   // device row counts: one pass (partials are sized by M)
+    // 64 x 64 tiles with a deep pipeline (gemm_small_kernel) where the
+    // 128 x 128 ones do not fill the chip.  Measured, 128 x 128 against
+    // 64 x 64 tiles (us): 256-k products, 100 tiles 27 / 17, 200 tiles
+    // 35 / 26, 400 tiles 47 / 43 with the K splits of the former and level at
+    // 190 tiles without them (24.5 / 25.1); 1 024 k, 24 tiles 23 / 20, 48
+    // tiles 27 / 29, 94 tiles 36 / 42, and over a device row count (no
+    // splits) 104 tiles 62 / 39, 160 tiles 63 / 42, 314 tiles 64 / 80; weight
+    // gradients of 3 000 rows, 4 tiles 24 / 14, 12 tiles 25 / 22, 16 tiles
+    // 25 / 25; of 10 000 rows, 4 tiles 24 / 23, 12 tiles 38 / 56.
+    if (!bf && vec && g.dma && dma_ok(g)) {
+        if (g.f32m) {
+            // the training forward keeps its splits: they are part of its rounding
+            g.small = tiles * splits <= cu;
+        } else if (g.a_t || (g.K > 512 && !g.Mdev)) {
+            g.small = (long)tiles * g.K < 44000;
+        } else {
+            g.small = tiles < 176;
+            if (!g.small && g.K <= 512) splits = 1;
+        }
+    }
+    if (g.small && !g.f32m) {
+        if (g.a_t) {
+            splits = pt_wgrad_splits(g.K, tiles_s, cu, bk, wsplit_ok);
+        } else {
+            splits = tiles_s < cu ? cu / tiles_s : 1;
+            if (splits > g.K / (16 * bk)) splits = g.K / (16 * bk);
+            if (splits < 1 || g.Mdev) splits = 1;
+        }
+    }
     // bf16 output products (GemmArgs::obf) never reach this path; every fp32
     // epilogue is applied by the reduce when K is split
     PT_REQUIRE(!(g.dbias && !(g.a_t && g.epi == EPI_STORE)), "gemm: dbias needs a_t = 1 and the STORE epilogue");
@@ -2699,7 +3464,7 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
         g.wsplit = cu;
         sdev = reinterpret_cast<const int*>(ws + (long)splits * per_split);
     }
-    dim3 grid(tn * tm, 1, splits);
+    dim3 grid(g.small ? tiles_s : tiles, 1, splits);
     if (bf && g.dbias && !db) {
         // bias sums first: they read the fp32 dY, which the product does not modify
         PT_TRY(pt_colsum(g.A, g.lda, g.K, g.M, g.dbias, ws, ws_floats, s));
@@ -2730,7 +3495,7 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
     // count (whole tiles and tail partials, then the partials' fixed-order
     // sums through the epilogue), where the host's row bound allows a tail
     // (S < T) and leaves fewer than 8 tiles per CU
-    if (g.Mdev && !g.Kdev && !db && !bf && g.dma && vec && ws != nullptr) {
+    if (g.Mdev && !g.Kdev && !db && !bf && g.dma && vec && !g.small && ws != nullptr) {
         const int S = pt_cu_count();
         if (S > 0 && tiles > S && tiles < 8 * S && (long)S * BM * BN <= ws_floats && try_dtail(g, tiles, S, ws, s)) {
             PT_LAUNCH_CHECK();
@@ -2742,7 +3507,7 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
     // the time).  Run the first T - T % S tiles whole and split the tail's K
     // across the idle CUs, then reduce the tail partials in a fixed order.
     // Worth its two extra launches only while a CU holds few tiles (T < 4 S).
-    if (!db && !g.Mdev && ws != nullptr) {
+    if (!db && !g.Mdev && !g.small && ws != nullptr) {
         const int S = pt_cu_count();
         const int R = S > 0 ? tiles % S : 0;
         const int ksteps = pt_cdiv(g.K, bk);

@@ -161,12 +161,22 @@ struct PtcgModel {
 };
 
 // ------------------------------------------------------------ helpers
+// The forward's products of a training step run on fp32 matrix instructions
+// (GemmArgs::f32m), the rollout's and the backward's on the three-way split,
+// which is faster and closer to 64 bits.  The gradient of score_mlp.2.bias is
+// a sum whose exact value is 0 (the softmax logits' gradients of a row cancel),
+// so what reaches the optimizer is the rounding of the logits, and Adam scales
+// it up by up to 1 / eps: another rounding of the forward moves every score of
+// the next step by up to 2e-5 of the output's norm (3 of 23 seeds above 1e-5
+// after one step), where the backward's moves it by below 1e-6.
+//
 // Y = epi(X W^T + b) with workspace ws for split-K / tail partials
 static int lin_ws(const PtcgModel* m, float* ws, long ws_floats, const float* X, long ldx, const float* W,
                   const float* b, float* Y, long ldy, int rows, int in, int out, int epi, const float* R, long ldr,
                   float* Y2, long ldy2, hipStream_t s, const int* Mdev = nullptr) {
     GemmArgs g{};
     g.prec = m->prec;
+    g.f32m = m->train;
     g.Mdev = Mdev;
     g.M = rows; g.N = out; g.K = in;
     g.A = X; g.lda = ldx; g.a_t = 0;
@@ -204,6 +214,7 @@ static int lin_resid_ln(const PtcgModel* m, const float* X, const float* W, cons
                         int in, int out, const float* R, const LnOut& ln, hipStream_t s, const int* Mdev) {
     GemmArgs g{};
     g.prec = m->prec;
+    g.f32m = m->train;
     g.Mdev = Mdev;
     g.M = rows; g.N = out; g.K = in;
     g.A = X; g.lda = in;

@@ -1,0 +1,122 @@
+"""fp32 products on the bf16 matrix pipe (three-way split of the operands):
+tile and k edges of the 128 x 128 and 64 x 64 kernels, non-finite and extreme
+operands, operands past 2^31 bytes, and the residual + LayerNorm forms.
+
+Tolerance: a 16-k step's products are summed exactly to 2^-26 and added to the
+fp32 accumulators once, so K / 16 roundings of 2^-24 (random signs) and the
+final one: relative L2 <= 2^-24 (2 + sqrt(K / 16)) against float64.  Split-K
+partials are summed in fp32, one more rounding per split (at most K / 16).
+"""
+import math
+
+import pytest
+import torch
+
+from conftest import rel_l2
+from ptcg_amd import native
+
+pytestmark = pytest.mark.gpu
+
+
+def bound(K):
+    return 2.0 ** -24 * (2 + math.sqrt(K / 16))
+
+
+def P(t):
+    return None if t is None else t.data_ptr()
+
+
+def gemm(A, B, M, N, K, a_t, b_t, epi=0, bias=None, R=None):
+    dA, dB = A.cuda().contiguous(), B.cuda().contiguous()
+    C, ws = torch.zeros(M, N, device="cuda"), torch.zeros(32 << 20, device="cuda")
+    native.check(native.lib().ptcg_kernel_gemm(M, N, K, P(dA), M if a_t else K, a_t, P(dB), N if b_t else K, b_t, P(C),
+                                               N, epi, P(bias), P(R), N, None, N, P(ws), ws.numel(), None))
+    torch.cuda.synchronize()
+    return C
+
+
+def operands(M, N, K, a_t, b_t, seed=0):
+    g = torch.Generator().manual_seed(seed + M * 7 + N * 3 + K)
+    A, B = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)
+    return A, B, (A.T if a_t else A), (B if b_t else B.T)
+
+
+# 64-tile kernel: tile and k-stage edges, fewer and more stages than its
+# pipeline; 128-tile kernel: the same and its balanced tail
+SHAPES = [(M, N, K) for M in (4, 60, 64, 68) for N, K in ((64, 4), (68, 12), (4, 132), (132, 1028))] + \
+         [(23000, 128, K) for K in (4, 16, 20, 300)] + [(33100, 132, 256), (22656, 64, 44), (128, 132, 9000)]
+
+
+@pytest.mark.parametrize("a_t,b_t", [(0, 0), (0, 1), (1, 1), (1, 0)])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_edges(M, N, K, a_t, b_t, cuda):
+    A, B, a, b = operands(M, N, K, a_t, b_t)
+    C = gemm(a, b, M, N, K, a_t, b_t)
+    ref = A.cuda().double() @ B.cuda().double()
+    assert rel_l2(C.cpu(), ref.cpu()) < bound(K), rel_l2(C.cpu(), ref.cpu())
+
+
+@pytest.mark.parametrize("M,N,K,a_t,b_t", [(100, 68, 64, 0, 0), (100, 68, 64, 1, 1), (23000, 128, 64, 0, 1)])
+def test_nonfinite(M, N, K, a_t, b_t, cuda):
+    """inf, -inf and NaN reach exactly the outputs they reach in float64
+    (no other operand element is 0, and no two of them meet)."""
+    A, B, _, _ = operands(M, N, K, a_t, b_t, seed=5)
+    A = A + torch.where(A < 0, -0.1, 0.1)
+    B = B + torch.where(B < 0, -0.1, 0.1)
+    A[3, 5], A[50, 9], B[7, 2] = math.inf, math.nan, -math.inf
+    C = gemm(A.T if a_t else A, B if b_t else B.T, M, N, K, a_t, b_t).cpu()
+    ref = (A.double() @ B.double()).float()
+    assert torch.equal(torch.isnan(C), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(C[inf], ref[inf]) and torch.equal(torch.isfinite(C), torch.isfinite(ref))
+    ok = torch.isfinite(ref)
+    assert rel_l2(C[ok], (A.double() @ B.double())[ok]) < 2.0 ** -24 * (2 + math.sqrt(K / 2))   # fp32 instructions
+
+
+@pytest.mark.parametrize("scale_a,scale_b", [(2.0 ** 100, 2.0 ** -90), (2.0 ** -100, 1.0), (2.0 ** -110, 2.0 ** 60),
+                                             (3.3e38, 2.0 ** -40)])
+def test_extremes(scale_a, scale_b, cuda):
+    """Operands near the ends of the fp32 range (finite values past the
+    largest bf16 among them)."""
+    M, N, K = 96, 64, 64
+    g = torch.Generator().manual_seed(9)
+    A = (0.5 + 0.53 * torch.rand(M, K, generator=g)).clamp(max=1.03) * torch.sign(torch.randn(M, K, generator=g))
+    A = (A.double() * scale_a).clamp(-3.4e38, 3.4e38).float()
+    B = (torch.randn(K, N, generator=g).double() * scale_b).float()
+    C = gemm(A, B.T, M, N, K, 0, 0)
+    ref = A.double() @ B.double()
+    assert rel_l2(C.cpu(), ref) < 2.0 ** -24 * (2 + math.sqrt(K / 2))
+
+
+def test_rows_past_2_31_bytes(cuda):
+    """A k-contiguous operand past 2^31 bytes: every row of the last tiles."""
+    M, N, K = 525000, 64, 1024
+    A = torch.randn(M, K, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    W = torch.randn(N, K, device="cuda", generator=torch.Generator("cuda").manual_seed(2))
+    C = torch.zeros(M, N, device="cuda")
+    native.check(native.lib().ptcg_kernel_gemm(M, N, K, P(A), K, 0, P(W), K, 0, P(C), N, 0, None, None, N, None, N,
+                                               None, 0, None))
+    torch.cuda.synchronize()
+    for rows in (slice(0, 300), slice(M - 600, M)):
+        ref = A[rows].double() @ W.double().T
+        assert rel_l2(C[rows].cpu(), ref.cpu()) < bound(K)
+
+
+@pytest.mark.parametrize("rows,K", [(1, 16), (31, 32), (33, 256), (8192, 64), (8193, 64), (20001, 256)])
+def test_resid_ln_equals_product_then_ln(rows, K, cuda):
+    """Both residual + LayerNorm forms (one 32-row tile per CU at most, and
+    64-row tiles) give the product's and the LayerNorm's bits."""
+    L = native.lib()
+    g = torch.Generator("cuda").manual_seed(rows + K)
+    f = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    A, W, bias, R, lw, lb = f(rows, K), f(256, K), f(256), f(rows, 256), f(256), f(256)
+    C, y, C2, y2 = (torch.zeros(rows, 256, device="cuda") for _ in range(4))
+    mu, rs, mu2, rs2 = (torch.zeros(rows, device="cuda") for _ in range(4))
+    native.check(L.ptcg_kernel_gemm_resid_ln(rows, K, P(A), P(W), P(bias), P(R), P(C), P(lw), P(lb), P(y), P(mu),
+                                             P(rs), 0, None, None))
+    native.check(L.ptcg_kernel_gemm(rows, 256, K, P(A), K, 0, P(W), K, 0, P(C2), 256, 3, P(bias), P(R), 256, None, 256,
+                                    None, 0, None))
+    native.check(L.ptcg_kernel_layernorm_fwd(P(C2), P(lw), P(lb), P(y2), P(mu2), P(rs2), rows, 256, None))
+    torch.cuda.synchronize()
+    for a, b in ((C, C2), (y, y2), (mu, mu2), (rs, rs2)):
+        assert torch.equal(a, b)
