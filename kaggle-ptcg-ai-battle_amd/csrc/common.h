@@ -129,16 +129,31 @@ __device__ __forceinline__ int pt_id_clamp(float v, int hi) {
     return i < 0 ? 0 : (i > hi ? hi : i);
 }
 
-// wave64 reductions (DPP/permute via __shfl_xor)
+// wave64 all-lane reductions over lane ^ 32, 16, 8, 4, 2, 1 in that order, on
+// register moves only: v_permlane32_swap / v_permlane16_swap bring the other
+// half / row, and within a row of 16 a rotation by 8, 4, 2, 1 reaches the same
+// value as the exclusive-or (after the step by 8 lanes i and i ^ 8 are equal,
+// and so on).  __shfl_xor goes through the LDS permute instruction, a round
+// trip per step: the LayerNorm epilogue of a lone 32 x 256 tile spent most of
+// its time in sixteen such chains.
+template <int N> __device__ __forceinline__ float row_ror(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true));
+}
+template <class Op> __device__ __forceinline__ float wave_reduce(float v, Op op) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    v = op(v, row_ror<8>(v));
+    v = op(v, row_ror<4>(v));
+    v = op(v, row_ror<2>(v));
+    return op(v, row_ror<1>(v));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return wave_reduce(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // row pointer of obs row n, optionally through an int32 row-index list

@@ -1558,31 +1558,44 @@ __device__ __forceinline__ void resid_ln_epilogue(const GemmArgs& g, const float
                 *reinterpret_cast<floatx4*>(smem + l32 * RL_SST + wn + 32 * tj + 8 * q + 4 * lh) =
                     floatx4{acc[h][tj][4 * q], acc[h][tj][4 * q + 1], acc[h][tj][4 * q + 2], acc[h][tj][4 * q + 3]};
         __syncthreads();
+        // four rows side by side: their wave sums do not depend on each other
+        // (rows past M are computed on R's first row and not stored)
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int lr = 8 * wave + r, m = m0 + 32 * h + lr;
-            if (m >= g.M) break;   // uniform over the wave; later rows are past M too
-            const floatx4 v = *reinterpret_cast<const floatx4*>(smem + lr * RL_SST + 4 * lane);
-            const floatx4 x = (v + bv) + rv[r];
-            st_g4(g.C + (long)m * g.ldc + 4 * lane, x);
-            const float mu = wave_sum((x[0] + x[1]) + (x[2] + x[3])) / (float)RL_N;
-            const float a = x[0] - mu, b = x[1] - mu, c = x[2] - mu, d = x[3] - mu;
-            const float var = wave_sum((a * a + b * b) + (c * c + d * d)) / (float)RL_N;
-            const float rs = 1.0f / sqrtf(var + 1e-5f);
-            if (lane == 0) {
-                mean[m] = mu;
-                rstd[m] = rs;
+        for (int r0 = 0; r0 < 8; r0 += 4) {
+            floatx4 x[4];
+            float mu[4], rs[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const floatx4 v = *reinterpret_cast<const floatx4*>(smem + (8 * wave + r0 + r) * RL_SST + 4 * lane);
+                x[r] = (v + bv) + rv[r0 + r];
+                mu[r] = wave_sum((x[r][0] + x[r][1]) + (x[r][2] + x[r][3])) / (float)RL_N;
             }
-            float4 o;
-            o.x = (x[0] - mu) * rs * ww.x + wb.x;
-            o.y = (x[1] - mu) * rs * ww.y + wb.y;
-            o.z = (x[2] - mu) * rs * ww.z + wb.z;
-            o.w = (x[3] - mu) * rs * ww.w + wb.w;
-            if constexpr (YB)
-                *reinterpret_cast<bf16x4*>(reinterpret_cast<__bf16*>(Y) + (long)m * ldy + 4 * lane) =
-                    bf16x4{(__bf16)o.x, (__bf16)o.y, (__bf16)o.z, (__bf16)o.w};
-            else
-                *reinterpret_cast<float4*>(Y + (long)m * ldy + 4 * lane) = o;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float a = x[r][0] - mu[r], b = x[r][1] - mu[r], c = x[r][2] - mu[r], d = x[r][3] - mu[r];
+                const float var = wave_sum((a * a + b * b) + (c * c + d * d)) / (float)RL_N;
+                rs[r] = 1.0f / sqrtf(var + 1e-5f);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = m0 + 32 * h + 8 * wave + r0 + r;
+                if (m >= g.M) break;   // uniform over the wave; later rows are past M too
+                st_g4(g.C + (long)m * g.ldc + 4 * lane, x[r]);
+                if (lane == 0) {
+                    mean[m] = mu[r];
+                    rstd[m] = rs[r];
+                }
+                float4 o;
+                o.x = (x[r][0] - mu[r]) * rs[r] * ww.x + wb.x;
+                o.y = (x[r][1] - mu[r]) * rs[r] * ww.y + wb.y;
+                o.z = (x[r][2] - mu[r]) * rs[r] * ww.z + wb.z;
+                o.w = (x[r][3] - mu[r]) * rs[r] * ww.w + wb.w;
+                if constexpr (YB)
+                    *reinterpret_cast<bf16x4*>(reinterpret_cast<__bf16*>(Y) + (long)m * ldy + 4 * lane) =
+                        bf16x4{(__bf16)o.x, (__bf16)o.y, (__bf16)o.z, (__bf16)o.w};
+                else
+                    *reinterpret_cast<float4*>(Y + (long)m * ldy + 4 * lane) = o;
+            }
         }
     }
 }
