@@ -179,6 +179,7 @@ enum PtEpi {
     EPI_BIAS_GELU_D = 6,  // z = acc + bias[n]; C = gelu'(z); C2 = gelu(z)
     EPI_MUL = 7,          // C = acc * R[m*ldr+n]
     EPI_AXPBY = 8,        // C = alpha * acc + beta * R[m*ldr+n] (alpha, beta in GemmArgs)
+    EPI_GELU = 9,         // C = gelu(acc + bias[n]): EPI_BIAS_GELU_D without a backward to keep gelu' for
 };
 
 struct GemmArgs {

@@ -101,6 +101,8 @@ __device__ __forceinline__ void epi_store_bf(const GemmArgs& g, int m, int n, fl
         pt_gelu_both_bf(v + g.bias[n], gv, gd);
         st_b1(g.C, c, gd);
         st_b1(g.C2, (long)m * g.ldc2 + n, gv);
+    } else if (EPI == EPI_GELU) {
+        st_b1(g.C, c, pt_gelu(v + g.bias[n]));
     } else if (EPI == EPI_MUL) {
         st_b1(g.C, c, v * ld_b1(g.R, (long)m * g.ldr + n));
     } else if (EPI == EPI_BIAS_RESID) {
@@ -130,6 +132,8 @@ __device__ __forceinline__ void epi_store(const GemmArgs& g, int m, int n, float
         pt_gelu_both(v + g.bias[n], gv, gd);
         g.C[(long)m * g.ldc + n] = gd;
         g.C2[(long)m * g.ldc2 + n] = gv;
+    } else if (EPI == EPI_GELU) {
+        g.C[(long)m * g.ldc + n] = pt_gelu(v + g.bias[n]);
     } else if (EPI == EPI_MUL) {
         g.C[(long)m * g.ldc + n] = v * g.R[(long)m * g.ldr + n];
     } else if (EPI == EPI_AXPBY) {
@@ -159,6 +163,9 @@ __device__ __forceinline__ void epi_store4_bf(const GemmArgs& g, int m, int n, f
         for (int i = 0; i < 4; ++i) pt_gelu_both_bf(v[i], gv[i], gd[i]);
         st_b4(g.C, c, floatx4{gd[0], gd[1], gd[2], gd[3]});
         st_b4(g.C2, (long)m * g.ldc2 + n, floatx4{gv[0], gv[1], gv[2], gv[3]});
+    } else if (EPI == EPI_GELU) {
+        v += ld_v4(g.bias + n);
+        st_b4(g.C, c, floatx4{pt_gelu(v[0]), pt_gelu(v[1]), pt_gelu(v[2]), pt_gelu(v[3])});
     } else if (EPI == EPI_MUL) {
         st_b4(g.C, c, v * ld_b4(g.R, (long)m * g.ldr + n));
     } else if (EPI == EPI_BIAS_RESID) {
@@ -192,6 +199,11 @@ __device__ __forceinline__ void epi_store8_bf(const GemmArgs& g, int m, int n, f
         }
         st_b8(g.C, c, floatx4{gd[0], gd[1], gd[2], gd[3]}, floatx4{gd[4], gd[5], gd[6], gd[7]});
         st_b8(g.C2, (long)m * g.ldc2 + n, floatx4{gv[0], gv[1], gv[2], gv[3]}, floatx4{gv[4], gv[5], gv[6], gv[7]});
+    } else if (EPI == EPI_GELU) {
+        v0 += ld_v4(g.bias + n);
+        v1 += ld_v4(g.bias + n + 4);
+        st_b8(g.C, c, floatx4{pt_gelu(v0[0]), pt_gelu(v0[1]), pt_gelu(v0[2]), pt_gelu(v0[3])},
+              floatx4{pt_gelu(v1[0]), pt_gelu(v1[1]), pt_gelu(v1[2]), pt_gelu(v1[3])});
     } else if (EPI == EPI_MUL) {
         const bf16x8s r = *(const gbf16x8*)(bfp(g.R) + (long)m * g.ldr + n);
         st_b8(g.C, c, v0 * floatx4{(float)r[0], (float)r[1], (float)r[2], (float)r[3]},
@@ -229,6 +241,9 @@ __device__ __forceinline__ void epi_store4(const GemmArgs& g, int m, int n, floa
         for (int i = 0; i < 4; ++i) pt_gelu_both(v[i], gv[i], gd[i]);
         st_g4(c, floatx4{gd[0], gd[1], gd[2], gd[3]});
         st_g4(g.C2 + (long)m * g.ldc2 + n, floatx4{gv[0], gv[1], gv[2], gv[3]});
+    } else if (EPI == EPI_GELU) {
+        v += ld_v4(g.bias + n);
+        st_g4(c, floatx4{pt_gelu(v[0]), pt_gelu(v[1]), pt_gelu(v[2]), pt_gelu(v[3])});
     } else if (EPI == EPI_MUL) {
         st_g4(c, v * ld_v4(g.R + (long)m * g.ldr + n));
     } else if (EPI == EPI_AXPBY) {
@@ -284,7 +299,7 @@ constexpr int SST = BN + 4;
 constexpr int STAGE_FLOATS = 64 * SST;
 template <int EPI> struct EpiStaged {
     static constexpr bool value = EPI == EPI_BIAS_GELU || EPI == EPI_GELU_BWD || EPI == EPI_BIAS_RESID ||
-                                  EPI == EPI_BIAS_GELU_D || EPI == EPI_MUL || EPI == EPI_AXPBY;
+                                  EPI == EPI_BIAS_GELU_D || EPI == EPI_GELU || EPI == EPI_MUL || EPI == EPI_AXPBY;
 };
 
 template <int EPI>
@@ -2726,6 +2741,7 @@ int launch_splitk_epi_reduce(const GemmArgs& g, const float* part, long part_str
         case EPI_BIAS_RESID: hipLaunchKernelGGL((splitk_epi_reduce_kernel<EPI_BIAS_RESID, V4>), gr, dim3(256), 0, s, g, part, part_stride, splits); break;
         case EPI_GELU_BWD: hipLaunchKernelGGL((splitk_epi_reduce_kernel<EPI_GELU_BWD, V4>), gr, dim3(256), 0, s, g, part, part_stride, splits); break;
         case EPI_BIAS_GELU_D: hipLaunchKernelGGL((splitk_epi_reduce_kernel<EPI_BIAS_GELU_D, V4>), gr, dim3(256), 0, s, g, part, part_stride, splits); break;
+        case EPI_GELU: hipLaunchKernelGGL((splitk_epi_reduce_kernel<EPI_GELU, V4>), gr, dim3(256), 0, s, g, part, part_stride, splits); break;
         case EPI_MUL: hipLaunchKernelGGL((splitk_epi_reduce_kernel<EPI_MUL, V4>), gr, dim3(256), 0, s, g, part, part_stride, splits); break;
         case EPI_AXPBY: hipLaunchKernelGGL((splitk_epi_reduce_kernel<EPI_AXPBY, V4>), gr, dim3(256), 0, s, g, part, part_stride, splits); break;
         default: PT_REQUIRE(false, "gemm: split-K epilogue %d not supported", g.epi);
@@ -2915,6 +2931,7 @@ int launch_bf16_epi(const GemmArgs& g, dim3 grid, int k_chunk, long part_stride,
         case EPI_BIAS_RESID: launch_bf16<AT, BT, EPI_BIAS_RESID, false, false>(g, grid, k_chunk, 0, s); break;
         case EPI_GELU_BWD: launch_bf16<AT, BT, EPI_GELU_BWD, false, false>(g, grid, k_chunk, 0, s); break;
         case EPI_BIAS_GELU_D: launch_bf16<AT, BT, EPI_BIAS_GELU_D, false, false>(g, grid, k_chunk, 0, s); break;
+        case EPI_GELU: launch_bf16<AT, BT, EPI_GELU, false, false>(g, grid, k_chunk, 0, s); break;
         case EPI_MUL: launch_bf16<AT, BT, EPI_MUL, false, false>(g, grid, k_chunk, 0, s); break;
         case EPI_AXPBY: launch_bf16<AT, BT, EPI_AXPBY, false, false>(g, grid, k_chunk, 0, s); break;
         case EPI_ACCUM: launch_bf16<AT, BT, EPI_ACCUM, false, false>(g, grid, k_chunk, 0, s); break;
@@ -2953,6 +2970,7 @@ int launch_epi(const GemmArgs& g, dim3 grid, int k_chunk, hipStream_t s) {
         case EPI_BIAS_RESID: launch<AT, BT, EPI_BIAS_RESID, false, false, VEC>(g, grid, k_chunk, 0, s); break;
         case EPI_GELU_BWD: launch<AT, BT, EPI_GELU_BWD, false, false, VEC>(g, grid, k_chunk, 0, s); break;
         case EPI_BIAS_GELU_D: launch<AT, BT, EPI_BIAS_GELU_D, false, false, VEC>(g, grid, k_chunk, 0, s); break;
+        case EPI_GELU: launch<AT, BT, EPI_GELU, false, false, VEC>(g, grid, k_chunk, 0, s); break;
         case EPI_MUL: launch<AT, BT, EPI_MUL, false, false, VEC>(g, grid, k_chunk, 0, s); break;
         case EPI_AXPBY: launch<AT, BT, EPI_AXPBY, false, false, VEC>(g, grid, k_chunk, 0, s); break;
         case EPI_ACCUM: launch<AT, BT, EPI_ACCUM, false, false, VEC>(g, grid, k_chunk, 0, s); break;
@@ -3121,6 +3139,7 @@ static int gemm_bs_nt(const GemmArgs& g, hipStream_t s) {
         case EPI_BIAS * 2 + 1: launch_bs<EPI_BIAS, true>(f, grid, s); break;
         case EPI_BIAS_RESID * 2: launch_bs<EPI_BIAS_RESID, false>(f, grid, s); break;
         case EPI_BIAS_GELU_D * 2 + 1: launch_bs<EPI_BIAS_GELU_D, true>(f, grid, s); break;
+        case EPI_GELU * 2 + 1: launch_bs<EPI_GELU, true>(f, grid, s); break;
         case EPI_MUL * 2 + 1: launch_bs<EPI_MUL, true>(f, grid, s); break;
         default:
             PT_REQUIRE(false, "gemm (bf16 operands): epilogue %d with %s output not built", g.epi,
@@ -3363,6 +3382,7 @@ static bool try_dtail(const GemmArgs& g, int tiles, int S, float* ws, hipStream_
         case EPI_BIAS: launch_dtail<false, false, EPI_BIAS>(g, tiles, S, ws, s); return true;
         case EPI_BIAS_RESID: launch_dtail<false, false, EPI_BIAS_RESID>(g, tiles, S, ws, s); return true;
         case EPI_BIAS_GELU_D: launch_dtail<false, false, EPI_BIAS_GELU_D>(g, tiles, S, ws, s); return true;
+        case EPI_GELU: launch_dtail<false, false, EPI_GELU>(g, tiles, S, ws, s); return true;
         default: return false;
     }
 }
@@ -3557,6 +3577,7 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
                 case EPI_BIAS_RESID: hipLaunchKernelGGL(tail_reduce_kernel<EPI_BIAS_RESID>, gr, dim3(256), 0, s, t, ws, s2); break;
                 case EPI_GELU_BWD: hipLaunchKernelGGL(tail_reduce_kernel<EPI_GELU_BWD>, gr, dim3(256), 0, s, t, ws, s2); break;
                 case EPI_BIAS_GELU_D: hipLaunchKernelGGL(tail_reduce_kernel<EPI_BIAS_GELU_D>, gr, dim3(256), 0, s, t, ws, s2); break;
+                case EPI_GELU: hipLaunchKernelGGL(tail_reduce_kernel<EPI_GELU>, gr, dim3(256), 0, s, t, ws, s2); break;
                 case EPI_MUL: hipLaunchKernelGGL(tail_reduce_kernel<EPI_MUL>, gr, dim3(256), 0, s, t, ws, s2); break;
                 case EPI_AXPBY: hipLaunchKernelGGL(tail_reduce_kernel<EPI_AXPBY>, gr, dim3(256), 0, s, t, ws, s2); break;
                 case EPI_ACCUM: hipLaunchKernelGGL(tail_reduce_kernel<EPI_ACCUM>, gr, dim3(256), 0, s, t, ws, s2); break;
