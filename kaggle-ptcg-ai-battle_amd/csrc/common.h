@@ -226,7 +226,8 @@ struct GemmArgs {
     // exact three-way split of the operands, at smaller error and higher rate).
     // k-contiguous operands only (the training forward, see model.hip).
     int f32m;
-    // set by pt_gemm: 64 x 64 tiles (gemm_small_kernel)
+    // set by pt_gemm: 1: 64 x 64 tiles (gemm_small_kernel), 2: 32 x 32 tiles,
+    // K over the workgroup's waves (gemm_ksplit_kernel)
     int small;
 };
 
@@ -265,6 +266,9 @@ __host__ __device__ inline int pt_split_chunks(int K, int splits, int bk, int* k
 // dims multiples of 4, 16 B-aligned bases.  Weight-gradient shapes
 // (large K, small M*N) are split over K with a deterministic reduction.
 int pt_gemm(const GemmArgs& g, float* splitk_ws, long splitk_ws_floats, hipStream_t s);
+// whether pt_gemm (with a workspace or a device row count) runs g on 32 x 32
+// tiles with K over a workgroup's waves
+bool pt_gemm_ksplit_fits(const GemmArgs& g);
 // C = A W^T + bias + R (N = 256; fp32 or, with g.bs, bf16 operands) and, in
 // the same launch, y = LayerNorm(C) with its mean / rstd (eps 1e-5; ybf: y in
 // bf16); pt_gemm_resid_ln_fits says whether g fits

@@ -1442,6 +1442,140 @@ __global__ __launch_bounds__(NT) void gemm_small_kernel(const GemmArgs g0, int k
     gemm_small_tile<AT, BT, EPI, PARTIAL, DB, F32M>(g0, k_chunk0, part_stride, blockIdx.x, blockIdx.z, gridDim.z, smem);
 }
 
+// ---------------------------------------------------------------- K split over a workgroup's waves
+// Where even the 64 x 64 tiles leave the chip to a chain of k stages (a
+// rollout of a few environments, a small minibatch's input gradients), a
+// workgroup takes a 32 x 32 tile and each of its eight waves an eighth of K:
+// the chain is K / 128 stages, and the waves' partial tiles meet in LDS, summed
+// in a fixed order by the epilogue.  Each wave stages its own operands by DMA,
+// two stages ahead in its own 8 KB of LDS, so the loop has no barrier (loads
+// straight to fragment registers touch one line per lane of a k-contiguous
+// operand and took 1.4 times as long).  Every element is split once per
+// 32 x 32 tile, more vector instructions than the larger tiles need, which
+// sets the upper end of its range (see pt_gemm).
+constexpr int KS_T = 32, KS_W = 8, KS_NT = 64 * KS_W, KS_LD = KS_T + 4;
+constexpr int KS_STAGE = 2 * KS_T * BK, KS_NS = 2, KS_WAVE = KS_NS * KS_STAGE;   // floats
+static_assert(KS_WAVE >= KS_T * KS_LD, "a wave's partial tile does not fit its stages");
+// LDS layouts of a 32 x 16 operand stage: [row][k] as the 64-row one's; [k][row]
+// takes k rows j and j + 8 side by side, which the two half waves of a fragment
+// read together, so they cover all banks
+template <bool T> __device__ __forceinline__ int ks_at(int r, int k) {
+    return T ? (2 * (k & 7) + (k >> 3)) * KS_T + r : small_at<false>(r, k);
+}
+// 1 KB DMA chunk c (0, 1) of a stage: 16 rows, or four pairs of k rows
+template <bool T> __device__ __forceinline__ int ks_src(int c, int lane, int r0, long ld) {
+    if (!T) return small_src<false>(c, lane, r0, ld);
+    const int p = 8 * c + (lane >> 3);
+    return (int)(((p >> 1) + 8 * (p & 1)) * ld) + r0 + 4 * (lane & 7);
+}
+template <bool T> __device__ __forceinline__ void ks_frag(const float* X, int l32, int lh, float (&x)[8]) {
+    if (!T) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float4 v = *reinterpret_cast<const float4*>(X + ks_at<false>(l32, 8 * lh + 4 * h));
+            x[4 * h] = v.x; x[4 * h + 1] = v.y; x[4 * h + 2] = v.z; x[4 * h + 3] = v.w;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = X[ks_at<true>(l32, 8 * lh + j)];
+    }
+}
+template <bool BT, int EPI>
+__global__ __launch_bounds__(KS_NT, 4) void gemm_ksplit_kernel(const GemmArgs g0) {
+    const GemmArgs g = gemm_shape(g0);
+    __shared__ __align__(16) float smem[KS_W * KS_WAVE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    int tmi, tni;
+    if (!tile_of_range<KS_T>(g, (g.N + KS_T - 1) / KS_T, tmi, tni, blockIdx.x)) return;   // beyond the tile count
+    const int m0 = tmi * KS_T, n0 = tni * KS_T;
+    const int chunk = ((g.K + KS_W * BK - 1) / (KS_W * BK)) * BK;
+    const int kbeg = wave * chunk, kend = min(g.K, kbeg + chunk);
+    const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
+    float* own = smem + wave * KS_WAVE;
+    floatx16 hi[1][1], lo[1];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) hi[0][0][e] = lo[0][e] = 0.f;
+    if (nk > 0) {   // uniform over the wave, and no barrier inside
+        // exact operand extents (host checked < 2^31 bytes)
+        const unsigned ea = (unsigned)((long)(g.M - 1) * g.lda + g.K) * 4u;
+        const unsigned eb = (unsigned)(BT ? ((long)(g.K - 1) * g.ldb + g.N) : ((long)(g.N - 1) * g.ldb + g.K)) * 4u;
+        const int32x4_t ra = buffer_rsrc(g.A, ea), rb = buffer_rsrc(g.B, eb);
+        const int sa0 = ks_src<false>(0, lane, m0, g.lda), sa1 = ks_src<false>(1, lane, m0, g.lda);
+        const int sb0 = ks_src<BT>(0, lane, n0, g.ldb), sb1 = ks_src<BT>(1, lane, n0, g.ldb);
+        const int kb = BT ? (int)g.ldb : 1;
+        auto issue = [&](int it) {
+            const int k0 = kbeg + it * BK;
+            const float* st = own + (it % KS_NS) * KS_STAGE;
+            dma16(ra, st, (sa0 + k0) * 4);
+            dma16(ra, st + 256, (sa1 + k0) * 4);
+            dma16(rb, st + KS_T * BK, (sb0 + k0 * kb) * 4);
+            dma16(rb, st + KS_T * BK + 256, (sb1 + k0 * kb) * 4);
+        };
+        issue(0);
+        if (nk > 1) issue(1);
+        for (int it = 0; it < nk; ++it) {
+            if (it + 1 < nk) wait_vm<4>();
+            else wait_vm<0>();
+            const float* st = own + (it % KS_NS) * KS_STAGE;
+            float a8[8], b8[8];
+            ks_frag<false>(st, l32, lh, a8);
+            ks_frag<BT>(st + KS_T * BK, l32, lh, b8);
+            const int kv = kend - (kbeg + it * BK);
+            if (kv < BK) {   // the row end inside the stage: what lies past it is not zero
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (8 * lh + j >= kv) a8[j] = b8[j] = 0.f;
+            }
+            if (it + KS_NS < nk) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the stage is read before it is overwritten
+                issue(it + KS_NS);
+            }
+            const Frag3 fa[1] = {split_frag(a8)};
+            mma_split(hi[0], lo, fa, split_frag(b8));
+        }
+        hi[0][0] += lo[0];
+        if (tile_nonfinite<1, 1>(hi)) {   // rare: this wave's K again on fp32 instructions
+#pragma unroll
+            for (int e = 0; e < 16; ++e) hi[0][0][e] = 0.f;
+            const int r = m0 + l32, c = n0 + l32;
+            for (int k0 = kbeg; k0 < kend; k0 += BK)
+                for (int j = 0; j < 8; ++j) {
+                    const int k = k0 + 8 * lh + j;
+                    const float av = r < g.M && k < kend ? g.A[(long)r * g.lda + k] : 0.f;
+                    const float bv = c < g.N && k < kend ? g.B[BT ? (long)k * g.ldb + c : (long)c * g.ldb + k] : 0.f;
+                    hi[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv, av, hi[0][0], 0, 0, 0);
+                }
+        }
+    }
+    // the partial tile over the wave's own stages (all landed and read)
+    float* P = own + l32 * KS_LD;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<floatx4*>(P + 8 * q + 4 * lh) =
+            floatx4{hi[0][0][4 * q], hi[0][0][4 * q + 1], hi[0][0][4 * q + 2], hi[0][0][4 * q + 3]};
+    __syncthreads();
+    if (tid >= KS_T * KS_T / 4) return;
+    const int r = tid / (KS_T / 4), c = 4 * (tid % (KS_T / 4)), m = m0 + r, n = n0 + c;
+    if (m >= g.M) return;
+    floatx4 v[KS_W];
+#pragma unroll
+    for (int w = 0; w < KS_W; ++w) v[w] = *reinterpret_cast<const floatx4*>(smem + w * KS_WAVE + r * KS_LD + c);
+#pragma unroll
+    for (int h = KS_W / 2; h > 0; h >>= 1)
+#pragma unroll
+        for (int w = 0; w < h; ++w) v[w] += v[w + h];
+    const uintptr_t al = (uintptr_t)g.C | (uintptr_t)g.C2 | (uintptr_t)g.R | (uintptr_t)g.bias |
+                         (uintptr_t)((g.ldc | g.ldc2 | g.ldr) * 4);
+    if ((al & 15) == 0 && n + 3 < g.N) {
+        epi_store4<EPI>(g, m, n, v[0]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < g.N) epi_store<EPI>(g, m, n + e, v[0][e]);
+    }
+}
+
 template <bool AT, bool BT, int EPI, bool PARTIAL, bool DB>
 __global__ __launch_bounds__(NT) void gemm_f32_dma_kernel(const GemmArgs g0, int k_chunk0, long part_stride) {
     __shared__ __align__(16) float smem[dma_smem_floats<DMA_NS>()];
@@ -2876,7 +3010,10 @@ double launch_flops(const GemmArgs& g) {
 template <bool AT, bool BT, int EPI, bool PARTIAL, bool DB, bool VEC>
 void launch(const GemmArgs& g, dim3 grid, int k_chunk, long part_stride, hipStream_t s) {
     const int slot = pt_prof_open(s);
-    if (VEC && g.dma && g.small) {
+    if (VEC && g.dma && g.small == 2) {
+        if constexpr (!AT && !PARTIAL && !DB)
+            hipLaunchKernelGGL((gemm_ksplit_kernel<BT, EPI>), grid, dim3(KS_NT), 0, s, g);
+    } else if (VEC && g.dma && g.small) {
         if (!g.f32m)
             hipLaunchKernelGGL((gemm_small_kernel<AT, BT, EPI, PARTIAL, DB, false>), grid, dim3(NT), 0, s, g, k_chunk,
                                part_stride);
@@ -3387,6 +3524,29 @@ static bool try_dtail(const GemmArgs& g, int tiles, int S, float* ws, hipStream_
     }
 }
 
+// Whether pt_gemm splits K over the waves of 32 x 32 tiles (gemm_ksplit_kernel;
+// callers without a workspace and with a host row count get the one-pass
+// order of sums instead).  Its time is its split instructions' (about 0.5 ns
+// per tile and stage of 16 k) plus the launch, the other kernels' below one
+// 128 x 128 tile per CU the chain of K / 16 stages, so the line lies higher
+// where K is long.  Measured, us, the former kernel (64 x 64 tiles, K splits
+// with a host row count) / this one: 1 200 x 256 x K 256 10.2 / 5.7 and
+// K 1 024 28.4 / 12.3 (host count 16.3 / 12.3); 2 000 x 768 x 256 (24 200 tile
+// stages) 14.5 / 13.7; 2 000 x 1 024 x 256 (32 300) 18.2 / 19.3; 7 000 x 256 x
+// 256 (28 000) 14.9 / 15.2; 7 000 x 256 x 768 (84 000) 32.3 / 29.1; 7 000 x
+// 256 x 1 024 (112 000) 41.6 / 39.0, host count 37.4 / 39.0.  Below 16 stages
+// the launch's workgroups count, hence the lower bound of 16.  A device row
+// count lies below the bound (a valid prefix of half to all positions), so its
+// line is a third higher.
+bool pt_gemm_ksplit_fits(const GemmArgs& g) {
+    if (g.prec == 1 || g.bs || g.f32m || g.a_t || g.Kdev || g.dbias || g.K % 4 != 0 || (g.b_t && g.N % 4 != 0) ||
+        g.lda % 4 != 0 || g.ldb % 4 != 0 || (((uintptr_t)g.A | (uintptr_t)g.B) & 15) != 0 || !dma_ok(g) || !split_ok(g))
+        return false;
+    const long steps = pt_cdiv(g.K, BK);
+    const long stages = (long)pt_cdiv(g.M, KS_T) * pt_cdiv(g.N, KS_T) * (steps > 16 ? steps : 16);
+    return stages <= (g.K > 512 ? 90000 : g.Mdev ? 32768 : 24576);
+}
+
 int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
     GemmArgs g = g0;
     PT_REQUIRE(g.M > 0 && g.N > 0 && g.K > 0, "gemm: empty shape %d x %d x %d", g.M, g.N, g.K);
@@ -3476,6 +3636,12 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
             if (splits < 1 || g.Mdev) splits = 1;
         }
     }
+    if (ws != nullptr || g.Mdev) {
+        if (pt_gemm_ksplit_fits(g)) {
+            g.small = 2;
+            splits = 1;
+        }
+    }
     // bf16 output products (GemmArgs::obf) never reach this path; every fp32
     // epilogue is applied by the reduce when K is split
     PT_REQUIRE(!(g.dbias && !(g.a_t && g.epi == EPI_STORE)), "gemm: dbias needs a_t = 1 and the STORE epilogue");
@@ -3497,7 +3663,7 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
         g.wsplit = cu;
         sdev = reinterpret_cast<const int*>(ws + (long)splits * per_split);
     }
-    dim3 grid(g.small ? tiles_s : tiles, 1, splits);
+    dim3 grid(g.small == 2 ? pt_cdiv(g.M, KS_T) * pt_cdiv(g.N, KS_T) : g.small ? tiles_s : tiles, 1, splits);
     if (bf && g.dbias && !db) {
         // bias sums first: they read the fp32 dY, which the product does not modify
         PT_TRY(pt_colsum(g.A, g.lda, g.K, g.M, g.dbias, ws, ws_floats, s));

@@ -221,7 +221,9 @@ struct LnOut {
 // 119 vs ~133, K 1024: 231 vs ~213.  In the CORE step (FFN2 at K 1024
 // unfused) +0.4% replayed, +0.8% stream-launched; the reference variant's
 // FFN2 at K 512 x 82.4k rows (280 vs ~258 alone) ran 0.3% slower unfused in
-// its step, so it stays fused.  Both give the same bits.
+// its step, so it stays fused.  Both give the same bits.  Few rows of a rollout
+// run apart as well, where the product takes 32 x 32 tiles with K over a
+// workgroup's waves (1 168 rows at K 256: 16.7 us fused, 6.3 + 4.7 apart).
 static int lin_resid_ln(const PtcgModel* m, const float* X, const float* W, const float* b, float* Y, int rows,
                         int in, int out, const float* R, const LnOut& ln, hipStream_t s, const int* Mdev) {
     GemmArgs g{};
@@ -234,7 +236,7 @@ static int lin_resid_ln(const PtcgModel* m, const float* X, const float* W, cons
     g.C = Y; g.ldc = out;
     g.bias = b; g.R = R; g.ldr = out;
     g.epi = EPI_BIAS_RESID;
-    if (pt_gemm_resid_ln_fits(g) && in < 1024)
+    if (pt_gemm_resid_ln_fits(g) && in < 1024 && !pt_gemm_ksplit_fits(g))
         return pt_gemm_resid_ln(g, ln.w, ln.b, ln.y, out, ln.mu, ln.rs, s, ln.ybf);
     PT_TRY(pt_gemm(g, m->ws, m->ws_floats, s));
     return pt_ln_fwd(Y, out, ln.w, ln.b, ln.y, out, ln.mu, ln.rs, rows, out, s, Mdev, ln.ybf);

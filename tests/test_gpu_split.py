@@ -1,5 +1,5 @@
 """fp32 products on the bf16 matrix pipe (three-way split of the operands):
-tile and k edges of the 128 x 128 and 64 x 64 kernels, non-finite and extreme
+tile and k edges of the 128 x 128, 64 x 64 and 32 x 32 kernels, non-finite and extreme
 operands, operands past 2^31 bytes, and the residual + LayerNorm forms.
 
 Tolerance: a 16-k step's products are summed exactly to 2^-26 and added to the
@@ -26,11 +26,13 @@ def P(t):
     return None if t is None else t.data_ptr()
 
 
-def gemm(A, B, M, N, K, a_t, b_t, epi=0, bias=None, R=None):
+def gemm(A, B, M, N, K, a_t, b_t, epi=0, bias=None, R=None, ws_floats=32 << 20):
+    """ws_floats 0: no workspace, so no K split of any kind."""
     dA, dB = A.cuda().contiguous(), B.cuda().contiguous()
-    C, ws = torch.zeros(M, N, device="cuda"), torch.zeros(32 << 20, device="cuda")
+    C, ws = torch.zeros(M, N, device="cuda"), torch.zeros(ws_floats, device="cuda")
     native.check(native.lib().ptcg_kernel_gemm(M, N, K, P(dA), M if a_t else K, a_t, P(dB), N if b_t else K, b_t, P(C),
-                                               N, epi, P(bias), P(R), N, None, N, P(ws), ws.numel(), None))
+                                               N, epi, P(bias), P(R), N, None, N, P(ws) if ws_floats else None, ws_floats,
+                                               None))
     torch.cuda.synchronize()
     return C
 
@@ -56,7 +58,23 @@ def test_edges(M, N, K, a_t, b_t, cuda):
     assert rel_l2(C.cpu(), ref.cpu()) < bound(K), rel_l2(C.cpu(), ref.cpu())
 
 
-@pytest.mark.parametrize("M,N,K,a_t,b_t", [(100, 68, 64, 0, 0), (100, 68, 64, 1, 1), (23000, 128, 64, 0, 1)])
+# the 64-tile kernel, and K over the waves of 32 x 32 tiles: row, column and k
+# edges, waves with no or a partial stage, more stages than are in flight
+@pytest.mark.parametrize("ws_floats", [0, 32 << 20])
+@pytest.mark.parametrize("b_t", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(1, 4, 4), (31, 36, 20), (33, 28, 124), (65, 132, 128), (100, 256, 132),
+                                   (300, 64, 664), (16, 32, 1028), (2000, 256, 960)])
+def test_small_grids(M, N, K, b_t, ws_floats, cuda):
+    A, B, a, b = operands(M, N, K, 0, b_t)
+    g = torch.Generator().manual_seed(M)
+    bias, R = torch.randn(N, generator=g).cuda(), torch.randn(M, N, generator=g).cuda()
+    C = gemm(a, b, M, N, K, 0, b_t, 3, bias, R, ws_floats)
+    ref = A.cuda().double() @ B.cuda().double() + bias.double() + R.double()
+    assert rel_l2(C.cpu(), ref.cpu()) < bound(K), rel_l2(C.cpu(), ref.cpu())
+
+
+@pytest.mark.parametrize("M,N,K,a_t,b_t", [(100, 68, 64, 0, 0), (100, 68, 64, 1, 1), (23000, 128, 64, 0, 1),
+                                             (100, 68, 160, 0, 1)])
 def test_nonfinite(M, N, K, a_t, b_t, cuda):
     """inf, -inf and NaN reach exactly the outputs they reach in float64
     (no other operand element is 0, and no two of them meet)."""
