@@ -6,7 +6,7 @@
 // At B samples these are five products of B rows (about 0.12 GFLOP at B =
 // 512): as separate GEMM launches they form a chain of ten or more dependent
 // launches whose latency, not their arithmetic, sets when the trunk can start.
-// Here a workgroup takes MC_R samples through all five layers with the
+// Here a workgroup takes one or four samples through all five layers with the
 // activations in LDS; each output element is a 16-lane group's fp32 dot
 // product (fused multiply-adds over each lane's k in order, then a fixed
 // butterfly over the group: deterministic), the weights read as contiguous
@@ -17,15 +17,18 @@
 
 namespace {
 
-constexpr int MC_R = 4;      // samples per workgroup
+// Samples per workgroup (template parameter R): four share each weight read
+// where every CU has a workgroup anyway; below that a workgroup takes one, a
+// quarter of the products in each of its dependent passes.
+constexpr int MC_RMAX = 4;
 constexpr int MC_T = 512;    // threads per workgroup
 constexpr int MC_LG = 16;    // lanes that split one column's k
 constexpr int MC_J = 4;      // columns per lane group and pass
 constexpr int MC_KB = 8;     // weight float4s per lane and column loaded together (k chunks of 512)
 constexpr int MC_COLS = MC_T / MC_LG * MC_J;   // columns per pass of the workgroup
-static_assert(MC_R <= MC_LG, "lane r of a group finishes row r");
+static_assert(MC_RMAX <= MC_LG, "lane r of a group finishes row r");
 
-// Z = X W^T + b for the workgroup's MC_R rows: X in LDS (MC_R x in, row
+// Z = X W^T + b for the workgroup's R rows: X in LDS (R x in, row
 // stride ldx), W (out, in) row-major.  Columns go MC_COLS at a time, MC_J to
 // each 16-lane group of the eight waves; the group's lanes split k (lane l of
 // the group takes float4s l, l + 16, ...: a group reads 256 contiguous bytes
@@ -36,6 +39,7 @@ static_assert(MC_R <= MC_LG, "lane r of a group finishes row r");
 // a lane, are all in flight at once.)  gelu: Y = gelu'(z), Y2 =
 // gelu(z), L = gelu(z); else Y = z, L = z.  Global rows past nrows are not
 // stored (their LDS rows are zeros in, finite values out).
+template <int MC_R>
 __device__ __forceinline__ void mc_dense(const float* X, int ldx, int in, const float* __restrict__ W, const float* __restrict__ b,
                          int out, bool gelu, float* __restrict__ Y, long ldy, float* __restrict__ Y2, long ldy2,
                          float* L, int ldl, int row0, int nrows) {
@@ -81,12 +85,17 @@ __device__ __forceinline__ void mc_dense(const float* X, int ldx, int in, const 
                 }
             }
         }
+        // over lane ^ 8, 4, 2, 1, as rotations of the row of 16 (see wave_reduce)
 #pragma unroll
-        for (int o = MC_LG / 2; o > 0; o >>= 1)
+        for (int c = 0; c < MC_J; ++c)
 #pragma unroll
-            for (int c = 0; c < MC_J; ++c)
-#pragma unroll
-                for (int r = 0; r < MC_R; ++r) acc[c][r] += __shfl_xor(acc[c][r], o, 64);
+            for (int r = 0; r < MC_R; ++r) {
+                float v = acc[c][r];
+                v += row_ror<8>(v);
+                v += row_ror<4>(v);
+                v += row_ror<2>(v);
+                acc[c][r] = v + row_ror<1>(v);
+            }
 #pragma unroll
         for (int c = 0; c < MC_J; ++c) {
             if (j[c] >= out) continue;
@@ -113,7 +122,8 @@ __device__ __forceinline__ void mc_dense(const float* X, int ldx, int in, const 
     }
 }
 
-// rows [row0, row0 + MC_R) of src (ld w) into LDS (MC_R x w), zeros past nrows
+// rows [row0, row0 + R) of src (ld w) into LDS (R x w), zeros past nrows
+template <int MC_R>
 __device__ void mc_load(float* dst, const float* __restrict__ src, int w, int row0, int nrows) {
     for (int i = threadIdx.x; i < MC_R * w; i += MC_T) {
         const int r = i / w, k = i - r * w;
@@ -121,6 +131,7 @@ __device__ void mc_load(float* dst, const float* __restrict__ src, int w, int ro
     }
 }
 
+template <int MC_R>
 __global__ __launch_bounds__(MC_T) void mlp_chain_fwd_kernel(const MlpChain a) {
     extern __shared__ __align__(16) float mc_smem[];
     const int lx = a.gf > a.din ? a.gf : a.din, lh = a.G > a.H ? a.G : a.H, bin = a.G + a.H;
@@ -130,26 +141,32 @@ __global__ __launch_bounds__(MC_T) void mlp_chain_fwd_kernel(const MlpChain a) {
     const int row0 = blockIdx.x * MC_R;
     const int nrows = a.N - row0 < MC_R ? a.N - row0 : MC_R;
     // global MLP
-    mc_load(xin, a.glob_in, a.gf, row0, nrows);
+    mc_load<MC_R>(xin, a.glob_in, a.gf, row0, nrows);
     __syncthreads();
-    mc_dense(xin, a.gf, a.gf, a.g1w, a.g1b, a.G, true, a.g1, a.G, a.g1a, a.G, hid, a.G, row0, nrows);
+    mc_dense<MC_R>(xin, a.gf, a.gf, a.g1w, a.g1b, a.G, true, a.g1, a.G, a.g1a, a.G, hid, a.G, row0, nrows);
     __syncthreads();
-    mc_dense(hid, a.G, a.G, a.g2w, a.g2b, a.G, false, a.gd, bin, nullptr, 0, gdl, bin, row0, nrows);
+    mc_dense<MC_R>(hid, a.G, a.G, a.g2w, a.g2b, a.G, false, a.gd, bin, nullptr, 0, gdl, bin, row0, nrows);
     __syncthreads();
     // decision MLP
-    mc_load(xin, a.dec_in, a.din, row0, nrows);
+    mc_load<MC_R>(xin, a.dec_in, a.din, row0, nrows);
     __syncthreads();
-    mc_dense(xin, a.din, a.din, a.d1w, a.d1b, a.H, true, a.d1, a.H, a.d1a, a.H, hid, a.H, row0, nrows);
+    mc_dense<MC_R>(xin, a.din, a.din, a.d1w, a.d1b, a.H, true, a.d1, a.H, a.d1a, a.H, hid, a.H, row0, nrows);
     __syncthreads();
-    mc_dense(hid, a.H, a.H, a.d2w, a.d2b, a.H, false, a.gd + a.G, bin, nullptr, 0, gdl + a.G, bin, row0, nrows);
+    mc_dense<MC_R>(hid, a.H, a.H, a.d2w, a.d2b, a.H, false, a.gd + a.G, bin, nullptr, 0, gdl + a.G, bin, row0, nrows);
     __syncthreads();
     // broadcast product over [g | d]
-    mc_dense(gdl, bin, bin, a.bcw, a.bcb, a.D, false, a.bc, a.D, nullptr, 0, nullptr, 0, row0, nrows);
+    mc_dense<MC_R>(gdl, bin, bin, a.bcw, a.bcb, a.D, false, a.bc, a.D, nullptr, 0, nullptr, 0, row0, nrows);
 }
 
-long mc_smem_bytes(const MlpChain& a) {
+// Up to one workgroup per CU of one sample each: forward at 16 samples 39.8 ->
+// 20.6 us, backward at 40 samples 65 -> 49 us; the whole step or rollout gains
+// up to 256 samples (step of 256: 4 766 -> 4 733 us).  The sums do not depend
+// on R.
+bool one_per_group(int n) { return n <= 256; }
+
+long mc_smem_bytes(const MlpChain& a, int R) {
     const int lx = a.gf > a.din ? a.gf : a.din, lh = a.G > a.H ? a.G : a.H;
-    return 4L * MC_R * (lx + lh + a.G + a.H);
+    return 4L * R * (lx + lh + a.G + a.H);
 }
 
 }  // namespace
@@ -159,7 +176,7 @@ bool pt_mlp_chain_fits(const MlpChain& a) {
     for (const float* p : w)
         if (p == nullptr || ((uintptr_t)p & 15) != 0) return false;
     return a.N >= 1 && a.gf % 4 == 0 && a.G % 4 == 0 && a.din % 4 == 0 && a.H % 4 == 0 && a.D >= 1 &&
-           mc_smem_bytes(a) <= 64 * 1024;
+           mc_smem_bytes(a, MC_RMAX) <= 64 * 1024;
 }
 
 int pt_mlp_chain_fwd(const MlpChain& a, hipStream_t s) {
@@ -168,7 +185,11 @@ int pt_mlp_chain_fwd(const MlpChain& a, hipStream_t s) {
     PT_REQUIRE(a.glob_in && a.dec_in && a.g1b && a.g2b && a.d1b && a.d2b && a.bcb && a.g1 && a.g1a && a.gd && a.d1 &&
                    a.d1a && a.bc,
                "mlp_chain: null pointer");
-    hipLaunchKernelGGL(mlp_chain_fwd_kernel, dim3(pt_cdiv(a.N, MC_R)), dim3(MC_T), (size_t)mc_smem_bytes(a), s, a);
+    if (one_per_group(a.N))
+        hipLaunchKernelGGL(mlp_chain_fwd_kernel<1>, dim3(a.N), dim3(MC_T), (size_t)mc_smem_bytes(a, 1), s, a);
+    else
+        hipLaunchKernelGGL(mlp_chain_fwd_kernel<MC_RMAX>, dim3(pt_cdiv(a.N, MC_RMAX)), dim3(MC_T),
+                           (size_t)mc_smem_bytes(a, MC_RMAX), s, a);
     PT_LAUNCH_CHECK();
     return PTCG_OK;
 }
@@ -176,21 +197,22 @@ int pt_mlp_chain_fwd(const MlpChain& a, hipStream_t s) {
 // The backward's dX products of the same chain in one launch (reference:
 // the autograd of ptcg/rl/model.py:223-235): dgd += dbc Wb, dd1 = (dgd[:, G:]
 // W4) * gelu'(z3), ddec = dd1 W3, dg1 = (dgd[:, :G] W2) * gelu'(z1).  A
-// workgroup takes MB_R samples; per product a thread owns an output column j
-// for all MB_R rows and runs over the reduction index in order (the weight
+// workgroup takes one or four samples; per product a thread owns an output
+// column j for all its rows and runs over the reduction index in order (the weight
 // row segments W[o][j..] of consecutive threads are contiguous), MB_B weights
 // in flight at once.  Deterministic; writes dgd, dd1, ddec and dg1 as the
 // separate products did.
 namespace {
 
-constexpr int MB_R = 4;      // samples per workgroup
+constexpr int MB_RMAX = 4;   // samples per workgroup (R), or one as in the forward
 constexpr int MB_T = 512;    // threads per workgroup
 constexpr int MB_B = 32;     // weights per thread loaded together
 
-// Y[r][j] (+)= sum_o X[r][o] W[o][j] for the workgroup's MB_R rows: X in LDS
-// (MB_R x nin at row stride ldx), W (nin, nout) row-major; mul: Y = sum *
+// Y[r][j] (+)= sum_o X[r][o] W[o][j] for the workgroup's R rows: X in LDS
+// (R x nin at row stride ldx), W (nin, nout) row-major; mul: Y = sum *
 // M[row][j] (M at row stride ldm); acc: Y = Yold + sum; L: the result for the
 // next product (LDS, row stride ldl)
+template <int MB_R>
 __device__ __forceinline__ void mb_dense(const float* X, int ldx, int nin, const float* __restrict__ W, int nout,
                                          float* __restrict__ Y, long ldy, bool acc, const float* __restrict__ M,
                                          long ldm, float* L, int ldl, int row0, int nrows) {
@@ -223,6 +245,7 @@ __device__ __forceinline__ void mb_dense(const float* X, int ldx, int nin, const
     }
 }
 
+template <int MB_R>
 __device__ __forceinline__ void mb_load(float* dst, int ldd, const float* __restrict__ src, long lds, int w, int row0,
                                         int nrows) {
     for (int i = threadIdx.x; i < MB_R * w; i += MB_T) {
@@ -231,6 +254,7 @@ __device__ __forceinline__ void mb_load(float* dst, int ldd, const float* __rest
     }
 }
 
+template <int MB_R>
 __global__ __launch_bounds__(MB_T) void mlp_chain_bwd_kernel(const MlpChainBwd a) {
     extern __shared__ __align__(16) float mb_smem[];
     const int bin = a.G + a.H;
@@ -239,17 +263,17 @@ __global__ __launch_bounds__(MB_T) void mlp_chain_bwd_kernel(const MlpChainBwd a
     float* dd1 = dgd + MB_R * bin;        // MB_R x H
     const int row0 = blockIdx.x * MB_R;
     const int nrows = a.N - row0 < MB_R ? a.N - row0 : MB_R;
-    mb_load(dbc, a.D, a.dbc, a.D, a.D, row0, nrows);
+    mb_load<MB_R>(dbc, a.D, a.dbc, a.D, a.D, row0, nrows);
     __syncthreads();
     // dgd += dbc Wb  (Wb: D x bin)
-    mb_dense(dbc, a.D, a.D, a.bcw, bin, a.dgd, bin, true, nullptr, 0, dgd, bin, row0, nrows);
+    mb_dense<MB_R>(dbc, a.D, a.D, a.bcw, bin, a.dgd, bin, true, nullptr, 0, dgd, bin, row0, nrows);
     __syncthreads();
     // dd1 = (dgd[:, G:] W4) * d1, W4: H x H;  dg1 = (dgd[:, :G] W2) * g1, W2: G x G
-    mb_dense(dgd + a.G, bin, a.H, a.d2w, a.H, a.dd1, a.H, false, a.d1, a.H, dd1, a.H, row0, nrows);
-    mb_dense(dgd, bin, a.G, a.g2w, a.G, a.dg1, a.G, false, a.g1, a.G, nullptr, 0, row0, nrows);
+    mb_dense<MB_R>(dgd + a.G, bin, a.H, a.d2w, a.H, a.dd1, a.H, false, a.d1, a.H, dd1, a.H, row0, nrows);
+    mb_dense<MB_R>(dgd, bin, a.G, a.g2w, a.G, a.dg1, a.G, false, a.g1, a.G, nullptr, 0, row0, nrows);
     __syncthreads();
     // ddec = dd1 W3, W3: H x din
-    mb_dense(dd1, a.H, a.H, a.d1w, a.din, a.ddec, a.din, false, nullptr, 0, nullptr, 0, row0, nrows);
+    mb_dense<MB_R>(dd1, a.H, a.H, a.d1w, a.din, a.ddec, a.din, false, nullptr, 0, nullptr, 0, row0, nrows);
 }
 
 }  // namespace
@@ -258,9 +282,12 @@ int pt_mlp_chain_bwd(const MlpChainBwd& a, hipStream_t s) {
     PT_REQUIRE(a.N >= 1 && a.G >= 1 && a.H >= 1 && a.din >= 1 && a.D >= 1, "mlp_chain_bwd: empty widths");
     PT_REQUIRE(a.dbc && a.bcw && a.g2w && a.d2w && a.d1w && a.g1 && a.d1 && a.dgd && a.dg1 && a.dd1 && a.ddec,
                "mlp_chain_bwd: null pointer");
-    const long smem = 4L * MB_R * (a.D + a.G + a.H + a.H);
+    const long smem = 4L * MB_RMAX * (a.D + a.G + a.H + a.H);
     PT_REQUIRE(smem <= 64 * 1024, "mlp_chain_bwd: widths %d / %d / %d exceed LDS", a.D, a.G, a.H);
-    hipLaunchKernelGGL(mlp_chain_bwd_kernel, dim3(pt_cdiv(a.N, MB_R)), dim3(MB_T), (size_t)smem, s, a);
+    if (one_per_group(a.N))
+        hipLaunchKernelGGL(mlp_chain_bwd_kernel<1>, dim3(a.N), dim3(MB_T), (size_t)smem / MB_RMAX, s, a);
+    else
+        hipLaunchKernelGGL(mlp_chain_bwd_kernel<MB_RMAX>, dim3(pt_cdiv(a.N, MB_RMAX)), dim3(MB_T), (size_t)smem, s, a);
     PT_LAUNCH_CHECK();
     return PTCG_OK;
 }
