@@ -1071,11 +1071,13 @@ template <bool T> struct SplitSlot {
     }
 };
 
-// A 128 x 128 tile of C by 4 waves of 64 x 64.  Each operand element is read to registers once per workgroup, split there and written to
-// LDS as three bf16 planes ([row][16 k], the two 16 B halves of a row swapped
-// every eight rows: conflict-free writes and fragment reads), two stages;
-// splitting at the fragment reads instead (fp32 in LDS by DMA) splits every
-// element twice.  A stage's loads are issued one stage ahead; one barrier per
+// A 128 x 128 tile of C by 4 waves of 64 x 64.  Each operand element is read
+// to registers once per workgroup, split there and written to LDS as three
+// bf16 planes ([row][16 k], the two 16 B halves of a row swapped every eight
+// rows: conflict-free writes and fragment reads), two stages; splitting at the fragment reads instead (fp32 in LDS by DMA) splits every
+// element twice.  Two stages of loads are in flight where A is k-contiguous, one
+// where it is transposed (see AHEAD; one: 149 504 x 256 x 1 024 500 us, two:
+// 458; x 768 x 256 423 and 404; 8192^3 5.92 and 5.45 ms); one barrier per
 // stage.  A transposed operand (weight gradients) is read row by row of k and
 // needs no transposition: the eight k of a slot are eight registers.
 // Same split-K, device-count, tail-partial and bias-sum rules as
@@ -1126,11 +1128,16 @@ __device__ __forceinline__ void gemm_split_tile(const GemmArgs& g0, int k_chunk0
     __bf16* sm = reinterpret_cast<__bf16*>(smem);
     const bool do_db = DB && AT && tni == 0;
     float dbsum = 0.f;
-    float xa[8], xb[8];
-    auto load = [&](int it) {   // past the last stage: out of range, zeros
+    struct Regs {
+        float a[8], b[8];
+    } x0, x1;
+    // stages in flight: two where the registers hold them, one where A is
+    // transposed too (sixteen 32-bit loads a stage)
+    constexpr int AHEAD = AT ? 1 : 2;
+    auto load = [&](int it, Regs& x) {   // past the last stage: out of range (zeros) or not used
         const int kv = kend - (kbeg + it * BK);
-        sa.load(it * BK, (int)g.lda, kv, xa);
-        sb.load(it * BK, (int)g.ldb, kv, xb);
+        sa.load(it * BK, (int)g.lda, kv, x.a);
+        sb.load(it * BK, (int)g.ldb, kv, x.b);
     };
     auto put = [&](__bf16* dst, const float (&x)[8], int r, int kg) {
         const Split8 f = split8(x);
@@ -1139,15 +1146,15 @@ __device__ __forceinline__ void gemm_split_tile(const GemmArgs& g0, int k_chunk0
         *reinterpret_cast<uint4*>(d + PLANE) = f.m;
         *reinterpret_cast<uint4*>(d + 2 * PLANE) = f.l;
     };
-    auto stage = [&](int it) {   // the loaded stage to LDS
+    auto stage = [&](int it, const Regs& x) {   // the loaded stage to LDS
         __bf16* st = sm + (it & 1) * STAGE;
-        put(st, xa, sa.r, sa.kg);
+        put(st, x.a, sa.r, sa.kg);
         if (DB && AT) {   // k rows past K were loaded as zeros; summed by every tile, a branch here would
                           // cut the loop body in two
 #pragma unroll
-            for (int j = 0; j < 8; ++j) dbsum += xa[j];
+            for (int j = 0; j < 8; ++j) dbsum += x.a[j];
         }
-        put(st + OPER, xb, sb.r, sb.kg);
+        put(st + OPER, x.b, sb.r, sb.kg);
     };
     auto frag = [&](const __bf16* plane, int row) {
         const __bf16* p = plane + split_at(row, lh);
@@ -1163,34 +1170,50 @@ __device__ __forceinline__ void gemm_split_tile(const GemmArgs& g0, int k_chunk0
         for (int tj = 0; tj < TT; ++tj) mma_split(acc[tj], low[tj], a, frag(st + OPER, wn + 32 * tj + l32));
     };
     if (nk > 0) {
-        load(0);
-        stage(0);
-        load(1);
-        __syncthreads();
-        for (int it = 0; it + 1 < nk; ++it) {   // branch-free: the splits fill the gaps between the products
+        auto body = [&](int it, Regs& x) {   // branch-free: the splits fill the gaps between the products
             mma(it);
-            stage(it + 1);   // the other buffer: its readers passed the last barrier
-            load(it + 2);
-            {
-                // issue order: fragments, then products with a few of the
-                // next stage's split instructions behind each (the matrix
-                // pipe is busy 32 cycles per product), LDS writes and the
-                // loads of the stage after it last
-                __builtin_amdgcn_sched_group_barrier(0x100, 9, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            stage(it + 1, x);   // the other buffer: its readers passed the last barrier
+            load(it + 1 + AHEAD, x);
+            // issue order: fragments, then products with a few of the next
+            // stage's split instructions behind each (the matrix pipe is busy
+            // 32 cycles per product), LDS writes and loads last
+            __builtin_amdgcn_sched_group_barrier(0x100, 9, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
 #pragma unroll
-                for (int i = 0; i < 18; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                }
-                __builtin_amdgcn_sched_group_barrier(0x200, 6, 0);
-                __builtin_amdgcn_sched_group_barrier(0x020, AT ? 16 : 4, 0);
+            for (int i = 0; i < 18; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             }
+            __builtin_amdgcn_sched_group_barrier(0x200, 6, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, AT ? 16 : 4, 0);
             __syncthreads();
+        };
+        int it = 0;
+        load(0, x0);
+        if constexpr (AHEAD == 2) {
+            load(1, x1);
+            stage(0, x0);
+            load(2, x0);
+            __syncthreads();
+            for (; it + 2 < nk; it += 2) {
+                body(it, x1);
+                body(it + 1, x0);
+            }
+            if (it + 1 < nk) {
+                mma(it);
+                stage(it + 1, x1);
+                __syncthreads();
+                ++it;
+            }
+        } else {
+            stage(0, x0);
+            load(1, x0);
+            __syncthreads();
+            for (; it + 1 < nk; ++it) body(it, x0);
         }
-        mma(nk - 1);
+        mma(it);
         __syncthreads();
     }
 #pragma unroll
