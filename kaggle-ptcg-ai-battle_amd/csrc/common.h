@@ -139,9 +139,8 @@ __device__ __forceinline__ int pt_id_clamp(float v, int hi) {
 template <int N> __device__ __forceinline__ float row_ror(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true));
 }
-template <class Op> __device__ __forceinline__ float wave_reduce(float v, Op op) {
-    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+// over lane ^ 16, 8, 4, 2, 1
+template <class Op> __device__ __forceinline__ float half_reduce(float v, Op op) {
     const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     v = op(__uint_as_float(b[0]), __uint_as_float(b[1]));
     v = op(v, row_ror<8>(v));
@@ -149,8 +148,17 @@ template <class Op> __device__ __forceinline__ float wave_reduce(float v, Op op)
     v = op(v, row_ror<2>(v));
     return op(v, row_ror<1>(v));
 }
+template <class Op> __device__ __forceinline__ float wave_reduce(float v, Op op) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return half_reduce(op(__uint_as_float(a[0]), __uint_as_float(a[1])), op);
+}
 __device__ __forceinline__ float wave_sum(float v) {
     return wave_reduce(v, [](float a, float b) { return a + b; });
+}
+// the sum of a product, its first step a fused multiply-add: own product
+// unrounded, the other half's rounded
+__device__ __forceinline__ float wave_sum_prod(float a, float b) {
+    return half_reduce(__builtin_fmaf(a, b, __shfl_xor(a * b, 32, 64)), [](float x, float y) { return x + y; });
 }
 __device__ __forceinline__ float wave_max(float v) {
     return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });

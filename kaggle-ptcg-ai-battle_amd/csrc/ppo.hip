@@ -107,7 +107,9 @@ __global__ __launch_bounds__(256) void ppo_loss_kernel(PPOArgs a) {
         const float lse = mx + logf(sum);
         const float logp = on ? l[j] - lse : 0.f;
         const float p = on ? expf(logp) : 0.f;
-        const float ent = -wave_sum(p * logp);
+        // (the rounding of this sum reaches the optimizer through
+        // score_mlp.2.bias, whose gradient is otherwise 0: see model.hip)
+        const float ent = -wave_sum_prod(p, logp);
         const float lp_act = __shfl(logp, act[j], 64);
         const float adv_n = (adv[j] - mean) / (adv_std + 1e-8f);
         // value loss + gradient (pufferlib.cu:1068-1085)
