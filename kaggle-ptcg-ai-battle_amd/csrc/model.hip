@@ -168,7 +168,8 @@ struct PtcgModel {
 // so what reaches the optimizer is the rounding of the logits, and Adam scales
 // it up by up to 1 / eps: another rounding of the forward moves every score of
 // the next step by up to 2e-5 of the output's norm (3 of 23 seeds above 1e-5
-// after one step), where the backward's moves it by below 1e-6.
+// after one step), where the backward's moves it by up to
+// 2e-6 (32 seeds).
 //
 // A GELU layer's forward keeps gelu'(z) for the backward (EPI_BIAS_GELU_D: Y
 // = gelu', Y2 = gelu); a rollout has none, so its layers write gelu(z) alone
