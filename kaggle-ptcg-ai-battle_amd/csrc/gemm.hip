@@ -3467,8 +3467,10 @@ int pt_gemm_resid_ln(const GemmArgs& g, const float* lnw, const float* lnb, floa
     } else {
         const dim3 grid(pt_cdiv(g.M, 32));
         // up to one 32-row tile per CU: six stages in flight (110 KB of LDS),
-        // a lone tile is bound by its chain of stages
-        const bool deep = (int)grid.x <= pt_cu_count();
+        // a lone tile is bound by its chain of stages.  Its DMA addresses the
+        // whole operand with 32-bit byte offsets (dma_ok; f32m operands passed
+        // that check above), the 64-row split kernel only a tile's rows.
+        const bool deep = (int)grid.x <= pt_cu_count() && dma_ok(g);
 #define PT_RLN(kernel, gr)                                                                                     \
     if (ybf) hipLaunchKernelGGL((kernel(true)), gr, blk, 0, s, f, lnw, lnb, y, ldy, mean, rstd);               \
     else hipLaunchKernelGGL((kernel(false)), gr, blk, 0, s, f, lnw, lnb, y, ldy, mean, rstd)

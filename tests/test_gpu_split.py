@@ -138,3 +138,25 @@ def test_resid_ln_equals_product_then_ln(rows, K, cuda):
     torch.cuda.synchronize()
     for a, b in ((C, C2), (y, y2), (mu, mu2), (rs, rs2)):
         assert torch.equal(a, b)
+
+
+def test_resid_ln_operand_past_2_32_bytes(cuda):
+    """Up to one 32-row tile per CU with an A whose extent does not fit 32
+    bits: rows from both ends, C and its LayerNorm (about a dozen fp32
+    roundings of 2^-24 after C)."""
+    rows, K = 8192, 131088
+    L = native.lib()
+    g = torch.Generator("cuda").manual_seed(3)
+    f = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    A, W, bias, R, lw, lb = f(rows, K), f(256, K), f(256), f(rows, 256), f(256), f(256)
+    C, y = torch.zeros(rows, 256, device="cuda"), torch.zeros(rows, 256, device="cuda")
+    mu, rs = torch.zeros(rows, device="cuda"), torch.zeros(rows, device="cuda")
+    native.check(L.ptcg_kernel_gemm_resid_ln(rows, K, P(A), P(W), P(bias), P(R), P(C), P(lw), P(lb), P(y), P(mu),
+                                             P(rs), 0, None, None))
+    torch.cuda.synchronize()
+    Wd = W.double().T.contiguous()
+    for sl in (slice(0, 33), slice(4090, 4100), slice(rows - 40, rows)):
+        ref = A[sl].double() @ Wd + bias.double() + R[sl].double()
+        assert rel_l2(C[sl].cpu(), ref.cpu()) < bound(K), rel_l2(C[sl].cpu(), ref.cpu())
+        ln = torch.nn.functional.layer_norm(C[sl].double(), (256,), lw.double(), lb.double(), 1e-5)
+        assert rel_l2(y[sl].cpu(), ln.cpu()) < 12 * 2.0 ** -24
