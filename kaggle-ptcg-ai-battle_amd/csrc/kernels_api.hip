@@ -124,6 +124,7 @@ extern "C" int ptcg_kernel_gemm_bs(int M, int N, int K, const void* A, int64_t l
                                    void* C, int64_t ldc, int epi, int out_bf16, const float* bias, const void* R,
                                    int64_t ldr, void* C2, int64_t ldc2, void* stream) {
     PT_REQUIRE(A && B && C, "kernel_gemm_bs: null operand");
+    PT_REQUIRE(epi >= EPI_STORE && epi <= EPI_MUL, "kernel_gemm_bs: bad epilogue %d", epi);
     PT_REQUIRE(!((epi == EPI_BIAS || epi == EPI_BIAS_RESID || epi == EPI_BIAS_GELU_D) && !bias),
                "kernel_gemm_bs: epilogue %d needs bias", epi);
     PT_REQUIRE(!((epi == EPI_BIAS_RESID || epi == EPI_MUL) && !R), "kernel_gemm_bs: epilogue %d needs R", epi);
