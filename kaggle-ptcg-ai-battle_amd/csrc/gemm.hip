@@ -959,9 +959,10 @@ __device__ __forceinline__ void gemm_dma_tile(const GemmArgs& g0, int k_chunk0, 
 // instruction (its clock drops with the operands' switching), so 290 for six,
 // against 155 for the fp32 one.
 // Denormal terms are kept by the instruction.  Inf and NaN do not survive the
-// split (inf - inf), nor do finite values past the largest bf16; they turn
-// every output of their row or column non-finite, which tile_nonfinite finds,
-// and the tile runs again on fp32 instructions.
+// split (inf - inf), nor do finite values past the largest bf16, and products
+// near the end of the range may overflow where their fp32 ones do not;
+// tile_nonfinite finds all of these in the outputs, and the tile runs again on
+// fp32 instructions.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 struct Split8 {
     uint4 h, m, l;   // eight bf16 each
@@ -1011,17 +1012,18 @@ __device__ __forceinline__ void mma_split(floatx16 (&hi)[TA], floatx16 (&lo)[TA]
     PT_SPLIT_TERM(lo, m, m) PT_SPLIT_TERM(lo, l, h) PT_SPLIT_TERM(lo, h, l)
 #undef PT_SPLIT_TERM
 }
-// whether the wave's tile holds an inf or NaN.  One in A's row reaches every
-// column of the row, one in B's column every row, so the registers of the
-// first row slice (all columns) and one register of every other slice do.
+// whether the wave's tile holds an inf or NaN.  Every register counts: an inf
+// or NaN operand reaches its whole row or column, but a product that
+// overflows only with its operands' leading terms rounded up, or a sum of
+// products that passes the fp32 range on the way, is one element's.
 template <int TA, int TB> __device__ __forceinline__ bool tile_nonfinite(const floatx16 (&acc)[TB][TA]) {
     float t = 0.f;
 #pragma unroll
     for (int tj = 0; tj < TB; ++tj)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) t = __builtin_fmaf(acc[tj][0][e], 0.f, t);
+        for (int ti = 0; ti < TA; ++ti)
 #pragma unroll
-    for (int ti = 1; ti < TA; ++ti) t = __builtin_fmaf(acc[0][ti][0], 0.f, t);
+            for (int e = 0; e < 16; ++e) t = __builtin_fmaf(acc[tj][ti][e], 0.f, t);
     return __builtin_amdgcn_ballot_w64(t != 0.f) != 0;
 }
 

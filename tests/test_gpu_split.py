@@ -106,6 +106,38 @@ def test_extremes(scale_a, scale_b, cuda):
     assert rel_l2(C.cpu(), ref) < 2.0 ** -24 * (2 + math.sqrt(K / 2))
 
 
+@pytest.mark.parametrize("M,K", [(100, 64), (23000, 64)])
+@pytest.mark.parametrize("m,n", [(0, 0), (40, 1), (33, 37), (95, 58)])
+def test_one_element_overflow(M, K, m, n, cuda):
+    """x y = 2^128 (1 - 2^-11)^2 is finite in fp32, its operands' leading bf16
+    terms (both 2^64) multiply to an infinity: one element of a tile, at any
+    of its registers (64- and 128-row tiles, both row and column slices)."""
+    N = 128
+    x = 2.0 ** 63 * (2 - 2.0 ** -10)
+    A, B = torch.zeros(M, K), torch.zeros(K, N)
+    A[m, 3], B[3, n] = x, x
+    C = gemm(A, B.T, M, N, K, 0, 0).cpu()
+    ref = (A.double() @ B.double()).float()
+    assert torch.isfinite(ref).all() and torch.equal(C, ref)
+
+
+@pytest.mark.parametrize("rows", [96, 8229])
+def test_resid_ln_one_element_overflow(rows, cuda):
+    """The same in both residual + LayerNorm forms (32- and 64-row tiles)."""
+    L, K = native.lib(), 64
+    x = 2.0 ** 63 * (2 - 2.0 ** -10)
+    A, W, R = (torch.zeros(s, device="cuda") for s in ((rows, K), (256, K), (rows, 256)))
+    A[45, 7], W[41, 7] = x, x
+    bias, lw, lb = (torch.zeros(256, device="cuda") for _ in range(3))
+    C, y, mu, rs = (torch.zeros(s, device="cuda") for s in ((rows, 256), (rows, 256), (rows,), (rows,)))
+    native.check(L.ptcg_kernel_gemm_resid_ln(rows, K, P(A), P(W), P(bias), P(R), P(C), P(lw), P(lb), P(y), P(mu),
+                                             P(rs), 0, None, None))
+    torch.cuda.synchronize()
+    ref = torch.zeros(rows, 256)
+    ref[45, 41] = 2.0 ** 127 * (2 - 2.0 ** -9 + 2.0 ** -21)
+    assert torch.equal(C.cpu(), ref)
+
+
 def test_rows_past_2_31_bytes(cuda):
     """A k-contiguous operand past 2^31 bytes: every row of the last tiles."""
     M, N, K = 525000, 64, 1024
