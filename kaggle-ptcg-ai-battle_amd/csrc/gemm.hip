@@ -958,12 +958,22 @@ __device__ __forceinline__ void gemm_dma_tile(const GemmArgs& g0, int k_chunk0, 
 // Rates measured on this GPU with random operands: 1 738 TFLOP/s for the bf16
 // instruction (its clock drops with the operands' switching), so 290 for six,
 // against 155 for the fp32 one.
-// Denormal terms are kept by the instruction.  Inf and NaN do not survive the
+// Denormal terms are kept by the instruction, and no fp32 operand is too small
+// (see SPLIT_UP).  Inf and NaN do not survive the
 // split (inf - inf), nor do finite values past the largest bf16, and products
 // near the end of the range may overflow where their fp32 ones do not;
 // tile_nonfinite finds all of these in the outputs, and the tile runs again on
 // fp32 instructions.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// Operands are split at 2^16 times their value: the smallest fp32 subnormal,
+// 2^-149, is then the smallest bf16 subnormal, so the three terms hold every
+// fp32 value exactly (unscaled, values below 2^-110 lose their low bits: 2^-9
+// of a value at 2^-126).  The sums are scaled back by 2^-32, exactly; what
+// passes the range by the scale alone (operands from 2^112, sums from 2^96)
+// reruns in fp32 with the other non-finite tiles.  The two multiplies per pair
+// beside eleven other instructions cost 1-2% of a rollout, a split weight
+// gradient or the Muon step, up to 13% of one small tile's long chain.
+constexpr float SPLIT_UP = 0x1p16f, SPLIT_DOWN = 0x1p-32f;
 struct Split8 {
     uint4 h, m, l;   // eight bf16 each
 };
@@ -983,7 +993,7 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
     unsigned h[4], m[4], l[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float a = x[2 * j], b = x[2 * j + 1];
+        const float a = SPLIT_UP * x[2 * j], b = SPLIT_UP * x[2 * j + 1];
         h[j] = pk_bf16(a, b);
         const float ra = a - __uint_as_float(h[j] << 16), rb = b - __uint_as_float(h[j] & mask);
         m[j] = pk_bf16(ra, rb);
@@ -1252,6 +1262,11 @@ __device__ __forceinline__ void gemm_split_tile(const GemmArgs& g0, int k_chunk0
                             acc[tj][ti] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[tj], av[ti], acc[tj][ti], 0, 0, 0);
                 }
             }
+        } else {
+#pragma unroll
+            for (int j = 0; j < TT; ++j)
+#pragma unroll
+                for (int i = 0; i < TT; ++i) acc[j][i] *= SPLIT_DOWN;
         }
     }
     if (DB && AT && do_db) {
@@ -1423,6 +1438,7 @@ __device__ __forceinline__ void gemm_small_tile(const GemmArgs& g0, int k_chunk0
         if (lane == 0) nonfinite[wave] = nf;
         __syncthreads();
         if (nonfinite[0] | nonfinite[1] | nonfinite[2] | nonfinite[3]) products(std::false_type{});   // rare
+        else hi[0][0] *= SPLIT_DOWN;
     }
     if (DB && AT && do_db) {
         __syncthreads();
@@ -1571,6 +1587,8 @@ __global__ __launch_bounds__(KS_NT, 4) void gemm_ksplit_kernel(const GemmArgs g0
                     const float bv = c < g.N && k < kend ? g.B[BT ? (long)k * g.ldb + c : (long)c * g.ldb + k] : 0.f;
                     hi[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv, av, hi[0][0], 0, 0, 0);
                 }
+        } else {
+            hi[0][0] *= SPLIT_DOWN;
         }
     }
     // the partial tile over the wave's own stages (all landed and read)
@@ -1921,6 +1939,9 @@ __global__ __launch_bounds__(NT) void gemm_resid_ln_kernel(const GemmArgs g0, co
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[0][j][e] = 0.f;
             products(std::false_type{});
+        } else {
+            acc[0][0] *= SPLIT_DOWN;
+            acc[0][1] *= SPLIT_DOWN;
         }
     }
     resid_ln_epilogue<YB, TM>(g, acc, m0, wave, lane, lnw, lnb, Y, ldy, mean, rstd, smem);
@@ -2031,6 +2052,11 @@ __global__ __launch_bounds__(NT, 2) void gemm_split_resid_ln_kernel(const GemmAr
                                 g.B[(long)(wn + 32 * tj + l32) * g.ldb + k], av, hi[tj][i], 0, 0, 0);
                     }
                 }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < TM; ++i) hi[j][i] *= SPLIT_DOWN;
         }
     }
     floatx16 acc[TM][2];

@@ -1,6 +1,6 @@
 """fp32 products on the bf16 matrix pipe (three-way split of the operands):
-tile and k edges of the 128 x 128, 64 x 64 and 32 x 32 kernels, non-finite and extreme
-operands, operands past 2^31 bytes, and the residual + LayerNorm forms.
+tile and k edges of the 128 x 128, 64 x 64 and 32 x 32 kernels, non-finite, extreme
+and tiny operands, operands past 2^31 bytes, and the residual + LayerNorm forms.
 
 Tolerance: a 16-k step's products are summed exactly to 2^-26 and added to the
 fp32 accumulators once, so K / 16 roundings of 2^-24 (random signs) and the
@@ -104,6 +104,56 @@ def test_extremes(scale_a, scale_b, cuda):
     C = gemm(A, B.T, M, N, K, 0, 0)
     ref = A.double() @ B.double()
     assert rel_l2(C.cpu(), ref) < 2.0 ** -24 * (2 + math.sqrt(K / 2))
+
+
+def tiny(M, K, e, seed):
+    """Random values of 2^e times [0.5, 1.03), rounded to fp32 (subnormals
+    below 2^-126)."""
+    g = torch.Generator().manual_seed(seed)
+    x = (0.5 + 0.53 * torch.rand(M, K, generator=g, dtype=torch.float64)) * torch.sign(torch.randn(M, K, generator=g))
+    return (x * 2.0 ** e).float()
+
+
+@pytest.mark.parametrize("M", [4, 96, 23000])   # 32 x 32, 64 x 64 (no workspace), 128 x 128 tiles
+@pytest.mark.parametrize("e", [-112, -118, -126, -133, -140])
+@pytest.mark.parametrize("a_t,b_t", [(0, 0), (1, 1)])
+def test_tiny_operands(M, e, a_t, b_t, cuda):
+    """Operands down to the fp32 subnormals keep all their bits against a
+    large partner, on either side."""
+    N, K = 128, 64
+    g = torch.Generator().manual_seed(1)
+    for swap in (False, True):
+        A = torch.randn(M, K, generator=g) * 2.0 ** 60 if swap else tiny(M, K, e, 2)
+        B = tiny(K, N, e, 3) if swap else torch.randn(K, N, generator=g) * 2.0 ** 60
+        C = gemm(A.T if a_t else A, B if b_t else B.T, M, N, K, a_t, b_t, ws_floats=0 if M == 96 else 32 << 20)
+        ref = A.double() @ B.double()
+        assert rel_l2(C.cpu(), ref) < bound(K), (swap, rel_l2(C.cpu(), ref))
+
+
+@pytest.mark.parametrize("rows", [96, 8229])
+def test_resid_ln_tiny_operands(rows, cuda):
+    """The same in both residual + LayerNorm forms."""
+    L, K = native.lib(), 64
+    g = torch.Generator().manual_seed(4)
+    A, W = tiny(rows, K, -126, 5).cuda(), (torch.randn(256, K, generator=g) * 2.0 ** 100).cuda()
+    bias, lw, lb = (torch.zeros(256, device="cuda") for _ in range(3))
+    R, C, y = (torch.zeros(rows, 256, device="cuda") for _ in range(3))
+    mu, rs = torch.zeros(rows, device="cuda"), torch.zeros(rows, device="cuda")
+    native.check(L.ptcg_kernel_gemm_resid_ln(rows, K, P(A), P(W), P(bias), P(R), P(C), P(lw), P(lb), P(y), P(mu),
+                                             P(rs), 0, None, None))
+    torch.cuda.synchronize()
+    ref = A.cpu().double() @ W.cpu().double().T
+    assert rel_l2(C.cpu(), ref) < bound(K)
+
+
+@pytest.mark.parametrize("M", [96, 23000])
+def test_sums_past_the_scaled_range(M, cuda):
+    """Sums of 2^110 pass the range of the scaled terms and run in fp32."""
+    N, K = 64, 64
+    A, B, _, _ = operands(M, N, K, 0, 0)
+    A, B = A * 2.0 ** 60, B * 2.0 ** 50
+    C = gemm(A, B.T, M, N, K, 0, 0)
+    assert rel_l2(C.cpu(), A.double() @ B.double()) < 2.0 ** -24 * (2 + math.sqrt(K / 2))   # fp32 instructions
 
 
 @pytest.mark.parametrize("M,K", [(100, 64), (23000, 64)])
