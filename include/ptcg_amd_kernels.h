@@ -29,6 +29,16 @@ int ptcg_kernel_gemm(int M, int N, int K, const float* A, int64_t lda, int a_t,
                      const float* bias, const float* R, int64_t ldr, float* C2, int64_t ldc2,
                      float* workspace, int64_t workspace_floats, void* stream);
 
+/* The kernel that ptcg_kernel_gemm (rows_dev = 0; workspace: whether one is
+ * given) or ptcg_kernel_gemm_rows_dev (rows_dev = 1) runs for 16 B aligned
+ * operands; train = 1: the training forward's form (fp32 matrix
+ * instructions).  0 register-staged (operands off the 128-bit or 2^31-byte
+ * rules), 1 128 x 128 tiles on fp32 matrix instructions, 2 128 x 128 tiles on
+ * the three-way bf16 split, 3 64 x 64 tiles, 4 32 x 32 tiles with K over a
+ * workgroup's waves.  Host only.                                            */
+int ptcg_kernel_gemm_path(int M, int N, int K, int64_t lda, int a_t, int64_t ldb, int b_t, int rows_dev,
+                          int workspace, int train);
+
 /* ptcg_kernel_gemm with a device row count, as the sync-free model's
  * launches run: M is the host's row bound, *rows_dev (device int, <= M) the
  * rows computed; rows past it are left alone.  A row-major A (a_t = 0) only;

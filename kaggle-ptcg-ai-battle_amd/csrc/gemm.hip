@@ -1042,7 +1042,8 @@ template <int TA, int TB> __device__ __forceinline__ bool tile_nonfinite(const f
 // load covers 64 consecutive floats of a k row; else at r ld + k, two 16 B
 // loads per slot.  Loads go through a buffer resource from the tile's first
 // row (a k-contiguous operand may thus pass 2^31 bytes) and stage to the
-// operand's end, clamped below 2^31 bytes: reads past it return zero.
+// operand's end, clamped 32 bytes below 2^31 (so that 0x7ffffff0 is past any):
+// reads past it return zero.
 template <bool T> struct SplitSlot {
     unsigned long long base;   // address of element (0, first row of the tile)
     int left;                  // floats from base to the operand's end
@@ -1058,7 +1059,7 @@ template <bool T> struct SplitSlot {
         const unsigned long long a = (unsigned long long)p;
         base = ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) |
                (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a);
-        left = __builtin_amdgcn_readfirstlane((int)(n < (1L << 29) - 1 ? n : (1L << 29) - 1));
+        left = __builtin_amdgcn_readfirstlane((int)(n < (1L << 29) - 8 ? n : (1L << 29) - 8));
     }
     // the stage at k (from the first): kv k are left of the chunk.  A
     // k-contiguous operand's row may end inside the stage (K a multiple of 4);
@@ -3279,16 +3280,16 @@ static bool dma_ok(const GemmArgs& g) {
            dma_fits(g.b_t ? g.K : g.N, g.b_t ? g.N : g.K, g.ldb);
 }
 
-// The split kernels rebase a k-contiguous operand at each tile's first row
-// (so only a tile's rows count) and a transposed one at the chunk's first k:
-// their offsets must stay below 2^31 bytes (2^29 floats, half of it for the
-// clamped extent)
-static bool split_fits(int rows, int cols, long ld, bool t) {
-    return t ? dma_fits(rows, cols, ld) : 2L * BM * ld + cols < (1L << 28);
+// The split kernels rebase a k-contiguous operand at each tile's first row, so
+// only a tile's rows count there (`tile`: the widest; 2^29 - 8 floats is the
+// longest extent, see SplitSlot, and loads run up to three stages past K), and a
+// transposed one at the chunk's first k.  Whatever dma_fits allows fits.
+static bool split_fits(int rows, int cols, long ld, bool t, int tile) {
+    return t ? dma_fits(rows, cols, ld) : tile * ld + cols < (1L << 29) - 64;
 }
-static bool split_ok(const GemmArgs& g) {
-    return split_fits(g.a_t ? g.K : g.M, g.a_t ? g.M : g.K, g.lda, g.a_t) &&
-           split_fits(g.b_t ? g.K : g.N, g.b_t ? g.N : g.K, g.ldb, g.b_t);
+static bool split_ok(const GemmArgs& g, int b_tile = BN) {
+    return split_fits(g.a_t ? g.K : g.M, g.a_t ? g.M : g.K, g.lda, g.a_t, BM) &&
+           split_fits(g.b_t ? g.K : g.N, g.b_t ? g.N : g.K, g.ldb, g.b_t, b_tile);
 }
 
 // ---- bf16 storage (GemmArgs::bs)
@@ -3468,7 +3469,7 @@ bool pt_gemm_resid_ln_fits(const GemmArgs& g) {
                          (uintptr_t)((g.lda | g.ldb) * (g.bs ? 2 : 4));
     const bool prec_ok = g.bs ? (g.K % 32 == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0) : (g.prec == 0 && g.K % BK == 0);
     return g.N == RL_N && g.M > 0 && prec_ok && !g.a_t && !g.b_t && g.epi == EPI_BIAS_RESID && !g.obf && g.bias &&
-           g.R && (al & 15) == 0 && !g.Kdev && (g.bs || g.f32m ? dma_ok(resid_ln_float_units(g)) : split_ok(g));
+           g.R && (al & 15) == 0 && !g.Kdev && (g.bs || g.f32m ? dma_ok(resid_ln_float_units(g)) : split_ok(g, RL_N));
 }
 int pt_gemm_resid_ln(const GemmArgs& g, const float* lnw, const float* lnb, float* y, long ldy, float* mean,
                      float* rstd, hipStream_t s, int ybf) {
@@ -3600,16 +3601,13 @@ bool pt_gemm_ksplit_fits(const GemmArgs& g) {
     return stages <= (g.K > 512 ? 90000 : g.Mdev ? 32768 : 24576);
 }
 
-int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
-    GemmArgs g = g0;
-    PT_REQUIRE(g.M > 0 && g.N > 0 && g.K > 0, "gemm: empty shape %d x %d x %d", g.M, g.N, g.K);
-    PT_REQUIRE(g.A && g.B && g.C, "gemm: null operand");
-    if (g.bs) {
-        PT_REQUIRE((!g.a_t && !g.b_t) || (g.a_t && g.b_t),
-                   "gemm (bf16 operands): A and B both k-contiguous or both transposed");
-        return g.a_t ? gemm_bs_dw(g, ws, ws_floats, s) : gemm_bs_nt(g, s);
-    }
-    PT_REQUIRE(!g.obf, "gemm: bf16 output needs bf16 operands");
+// How a product on fp32-stored operands runs: the operand path, the kernel
+// (g.dma, g.small) and the K splits before the workspace bounds them.
+struct GemmPlan {
+    bool vec, bf, wsplit_ok;
+    int bk, cu, tiles, tiles_s, splits;
+};
+static GemmPlan gemm_plan(GemmArgs& g, bool have_ws) {
     // 128-bit loads need the contiguous extent and the leading dimensions to be
     // multiples of 4 floats and 16 B aligned operands; otherwise scalar loads
     const bool vec = (g.a_t ? (g.M % 4 == 0) : (g.K % 4 == 0)) && (g.b_t ? (g.N % 4 == 0) : (g.K % 4 == 0)) &&
@@ -3617,7 +3615,6 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
                      ((uintptr_t)g.B & 15) == 0;
     // bf16 products need the 128-bit operand path; other shapes stay fp32
     const bool bf = g.prec == 1 && vec;
-    PT_REQUIRE(!g.f32m || (!g.a_t && !g.b_t), "gemm: fp32 instructions need k-contiguous operands");
     g.dma = vec && (bf || g.f32m ? dma_ok(g) : split_ok(g));
     const int bk = bf && !g.dma ? BK2 : BK;
     const int tm = pt_cdiv(g.M, BM), tn = pt_cdiv(g.N, BN);
@@ -3689,12 +3686,49 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
             if (splits < 1 || g.Mdev) splits = 1;
         }
     }
-    if (ws != nullptr || g.Mdev) {
+    if (have_ws || g.Mdev) {
         if (pt_gemm_ksplit_fits(g)) {
             g.small = 2;
             splits = 1;
         }
     }
+    return GemmPlan{vec, bf, wsplit_ok, bk, cu, tiles, tiles_s, splits};
+}
+
+// ptcg_kernel_gemm_path's codes
+enum GemmPath { PATH_REG = 0, PATH_F32 = 1, PATH_SPLIT = 2, PATH_SMALL = 3, PATH_KSPLIT = 4 };
+extern "C" int ptcg_kernel_gemm_path(int M, int N, int K, int64_t lda, int a_t, int64_t ldb, int b_t, int rows_dev,
+                                     int workspace, int train) {
+    PT_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_path: empty shape %d x %d x %d", M, N, K);
+    PT_REQUIRE(!train || (!a_t && !b_t), "gemm_path: the training forward's operands are k-contiguous");
+    GemmArgs g{};
+    g.M = M; g.N = N; g.K = K;
+    g.lda = lda; g.a_t = a_t;
+    g.ldb = ldb; g.b_t = b_t;
+    g.f32m = train;
+    const int count = 0;
+    if (rows_dev) g.Mdev = &count;   // not read
+    const GemmPlan p = gemm_plan(g, workspace != 0);
+    if (!p.vec || !g.dma) return PATH_REG;
+    if (g.small) return g.small == 2 ? PATH_KSPLIT : PATH_SMALL;
+    return g.f32m ? PATH_F32 : PATH_SPLIT;
+}
+
+int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
+    GemmArgs g = g0;
+    PT_REQUIRE(g.M > 0 && g.N > 0 && g.K > 0, "gemm: empty shape %d x %d x %d", g.M, g.N, g.K);
+    PT_REQUIRE(g.A && g.B && g.C, "gemm: null operand");
+    if (g.bs) {
+        PT_REQUIRE((!g.a_t && !g.b_t) || (g.a_t && g.b_t),
+                   "gemm (bf16 operands): A and B both k-contiguous or both transposed");
+        return g.a_t ? gemm_bs_dw(g, ws, ws_floats, s) : gemm_bs_nt(g, s);
+    }
+    PT_REQUIRE(!g.obf, "gemm: bf16 output needs bf16 operands");
+    PT_REQUIRE(!g.f32m || (!g.a_t && !g.b_t), "gemm: fp32 instructions need k-contiguous operands");
+    const GemmPlan plan = gemm_plan(g, ws != nullptr);
+    const bool vec = plan.vec, bf = plan.bf, wsplit_ok = plan.wsplit_ok;
+    const int bk = plan.bk, cu = plan.cu, tiles = plan.tiles, tiles_s = plan.tiles_s;
+    int splits = plan.splits;
     // bf16 output products (GemmArgs::obf) never reach this path; every fp32
     // epilogue is applied by the reduce when K is split
     PT_REQUIRE(!(g.dbias && !(g.a_t && g.epi == EPI_STORE)), "gemm: dbias needs a_t = 1 and the STORE epilogue");

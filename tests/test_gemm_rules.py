@@ -15,3 +15,35 @@ def test_bs_refuses_internal_epilogues(epi, out_bf16):
     with pytest.raises(native.PtcgError, match="epilogue"):
         native.check(native.lib().ptcg_kernel_gemm_bs(64, 64, 64, PTR, 64, PTR, 64, PTR, 64, epi, out_bf16, None, None,
                                                       64, None, 64, None))
+
+
+REG, F32, SPLIT, SMALL, KSPLIT = range(5)
+
+
+def path(M, N, K, lda=None, a_t=0, ldb=None, b_t=0, rows_dev=0, ws=1, train=0):
+    return native.lib().ptcg_kernel_gemm_path(M, N, K, lda or (M if a_t else K), a_t, ldb or (N if b_t else K), b_t,
+                                              rows_dev, ws, train)
+
+
+@pytest.mark.parametrize("M,N,K", [(4, 4, 1500000), (16, 64, 1200000), (300, 4, 900000)])
+@pytest.mark.parametrize("ws", [0, 1])
+def test_long_rows_stay_on_the_dma_kernels(M, N, K, ws):
+    """k-contiguous operands within the 2^31-byte rules of the DMA kernels
+    (tile rows past the end counted) never fall to the register-staged one."""
+    assert (max(M, N) + 256) * K + K + 256 < 1 << 29
+    assert path(M, N, K, ws=ws) in (SPLIT, SMALL, KSPLIT)
+    assert path(M, N, K, ws=ws, train=1) in (F32, SMALL)
+
+
+def test_rows_past_2_31_bytes_run_the_split():
+    assert path(525000, 64, 1024) == SPLIT
+    assert path(525000, 64, 1024, train=1) == REG
+    assert path(128, 128, 1 << 23) == REG
+
+
+@pytest.mark.parametrize("a_t,b_t", [(0, 0), (0, 1), (1, 1), (1, 0)])
+def test_operands_off_the_128_bit_rules(a_t, b_t):
+    M, N, K = (127, 64, 64) if a_t else (64, 64, 127)
+    assert path(M, N, K, a_t=a_t, b_t=b_t) == REG
+    assert path(64, 64, 64, lda=65, a_t=a_t, b_t=b_t) == REG
+    assert path(64, 64, 64, a_t=a_t, b_t=b_t) != REG

@@ -202,6 +202,17 @@ def test_rows_past_2_31_bytes(cuda):
         assert rel_l2(C[rows].cpu(), ref.cpu()) < bound(K)
 
 
+@pytest.mark.parametrize("ws_floats", [0, 32 << 20])
+@pytest.mark.parametrize("M,N,K", [(4, 4, 1500000), (130, 68, 1000000)])
+def test_long_rows(M, N, K, ws_floats, cuda):
+    """Rows of 2^20 floats and more: tile rows past the end lie past 2^28
+    floats.  K / 16 roundings in one chain without a workspace."""
+    A = torch.randn(M, K, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    W = torch.randn(N, K, device="cuda", generator=torch.Generator("cuda").manual_seed(2))
+    C = gemm(A, W, M, N, K, 0, 0, ws_floats=ws_floats)
+    assert rel_l2(C.cpu(), (A.double() @ W.double().T).cpu()) < bound(K)
+
+
 @pytest.mark.parametrize("rows,K", [(1, 16), (31, 32), (33, 256), (8192, 64), (8193, 64), (20001, 256)])
 def test_resid_ln_equals_product_then_ln(rows, K, cuda):
     """Both residual + LayerNorm forms (one 32-row tile per CU at most, and
