@@ -3591,11 +3591,16 @@ static bool try_dtail(const GemmArgs& g, int tiles, int S, float* ws, hipStream_
 // 256 x 1 024 (112 000) 41.6 / 39.0, host count 37.4 / 39.0.  Below 16 stages
 // the launch's workgroups count, hence the lower bound of 16.  A device row
 // count lies below the bound (a valid prefix of half to all positions), so its
-// line is a third higher.
+// line is a third higher.  However few the tiles, a wave walks K / 128 stages in
+// turn: past K 2 048 (a wave's 16) a host row count's K splits over the chip are
+// faster (32 x 32 outputs: K 1 536 9.1 here against 12.7, K 2 048 11.1 / 12.0,
+// K 3 072 15.1 / 12.8, K 16 384 60 / 25; 300 x 256: K 2 048 11.9 / 13.5, K 4 096
+// 22.0 / 17.9), a device row count has none and stays.
 bool pt_gemm_ksplit_fits(const GemmArgs& g) {
     if (g.prec == 1 || g.bs || g.f32m || g.a_t || g.Kdev || g.dbias || g.K % 4 != 0 || (g.b_t && g.N % 4 != 0) ||
         g.lda % 4 != 0 || g.ldb % 4 != 0 || (((uintptr_t)g.A | (uintptr_t)g.B) & 15) != 0 || !dma_ok(g) || !split_ok(g))
         return false;
+    if (!g.Mdev && g.K > 2048) return false;
     const long steps = pt_cdiv(g.K, BK);
     const long stages = (long)pt_cdiv(g.M, KS_T) * pt_cdiv(g.N, KS_T) * (steps > 16 ? steps : 16);
     return stages <= (g.K > 512 ? 90000 : g.Mdev ? 32768 : 24576);

@@ -47,3 +47,16 @@ def test_operands_off_the_128_bit_rules(a_t, b_t):
     assert path(M, N, K, a_t=a_t, b_t=b_t) == REG
     assert path(64, 64, 64, lda=65, a_t=a_t, b_t=b_t) == REG
     assert path(64, 64, 64, a_t=a_t, b_t=b_t) != REG
+
+
+@pytest.mark.parametrize("M,N", [(4, 4), (36, 128), (300, 256), (2000, 256)])
+@pytest.mark.parametrize("b_t", [0, 1])
+def test_long_k_is_split_over_the_chip(M, N, b_t):
+    """K over one workgroup's waves ends where the chain of a wave's stages
+    (K / 128) costs more than K splits over the chip and their reduce; a
+    device row count has no K splits."""
+    for K in (256, 1024, 2048):
+        assert path(M, N, K, b_t=b_t) == KSPLIT
+    for K in (2052, 4096, 16384, 1 << 20):
+        assert path(M, N, K, b_t=b_t) in (SMALL, SPLIT)
+    assert path(M, N, 4096, b_t=b_t, rows_dev=1) == (KSPLIT if M < 2000 else SMALL)
