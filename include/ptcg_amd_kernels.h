@@ -33,8 +33,8 @@ int ptcg_kernel_gemm(int M, int N, int K, const float* A, int64_t lda, int a_t,
  * given) or ptcg_kernel_gemm_rows_dev (rows_dev = 1) runs for 16 B aligned
  * operands; train = 1: the training forward's form (fp32 matrix
  * instructions).  0 register-staged (operands off the 128-bit or 2^31-byte
- * rules), 1 128 x 128 tiles on fp32 matrix instructions, 2 128 x 128 tiles on
- * the three-way bf16 split, 3 64 x 64 tiles, 4 32 x 32 tiles with K over a
+ * rules), 1 128 x 128 tiles on fp32 matrix instructions (the training forward,
+ * short K), 2 128 x 128 tiles on the three-way bf16 split, 3 64 x 64 tiles, 4 32 x 32 tiles with K over a
  * workgroup's waves.  Host only.                                            */
 int ptcg_kernel_gemm_path(int M, int N, int K, int64_t lda, int a_t, int64_t ldb, int b_t, int rows_dev,
                           int workspace, int train);

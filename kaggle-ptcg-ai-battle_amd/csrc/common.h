@@ -232,7 +232,8 @@ struct GemmArgs {
     int wsplit;
     // fp32 products on the fp32 matrix instructions (0: on the bf16 pipe by an
     // exact three-way split of the operands, at smaller error and higher rate).
-    // k-contiguous operands only (the training forward, see model.hip).
+    // Callers set it for k-contiguous operands only (the training forward, see
+    // model.hip); pt_gemm for products of one to three k stages on wide grids.
     int f32m;
     // set by pt_gemm: 1: 64 x 64 tiles (gemm_small_kernel), 2: 32 x 32 tiles,
     // K over the workgroup's waves (gemm_ksplit_kernel)

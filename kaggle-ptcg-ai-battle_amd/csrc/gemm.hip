@@ -3076,8 +3076,9 @@ void launch(const GemmArgs& g, dim3 grid, int k_chunk, long part_stride, hipStre
         hipLaunchKernelGGL((gemm_split_kernel<AT, BT, EPI, PARTIAL, DB>), grid, dim3(NT), 0, s, g, k_chunk,
                            part_stride);
     } else if (VEC && g.dma) {
-        // the training forward's layouts
-        if constexpr (!AT && !BT)
+        // the training forward's products and short K (no split-K form with a
+        // transposed operand)
+        if constexpr (!PARTIAL || (!AT && !BT))
             hipLaunchKernelGGL((gemm_f32_dma_kernel<AT, BT, EPI, PARTIAL, DB>), grid, dim3(NT), 0, s, g, k_chunk,
                                part_stride);
     } else
@@ -3609,7 +3610,7 @@ bool pt_gemm_ksplit_fits(const GemmArgs& g) {
 // How a product on fp32-stored operands runs: the operand path, the kernel
 // (g.dma, g.small) and the K splits before the workspace bounds them.
 struct GemmPlan {
-    bool vec, bf, wsplit_ok;
+    bool vec, bf, wsplit_ok, tail;
     int bk, cu, tiles, tiles_s, splits;
 };
 static GemmPlan gemm_plan(GemmArgs& g, bool have_ws) {
@@ -3691,13 +3692,33 @@ static GemmPlan gemm_plan(GemmArgs& g, bool have_ws) {
             if (splits < 1 || g.Mdev) splits = 1;
         }
     }
+    // A few k stages on a wide grid: bound by the outputs and by how many
+    // workgroups fit a CU, four of the fp32 instructions' kernel against two of
+    // the split's 128 x 128 or 64 x 64 tiles.  Measured, us, split / fp32
+    // instructions: bias + residual at K 16, 516 tiles (the split's second
+    // round of workgroups) 22.8 / 17.9, 752 tiles 24.6 / 21.0, 3 126 tiles
+    // 101 / 98, but 440 tiles 15.4 / 15.2 and 314 tiles 12.5 / 12.5; at K 48
+    // 516 tiles 24.8 / 22.8, 1 064 tiles 37.4 / 40.5; a GELU's longer epilogue
+    // at K 48, 1 563 tiles 51.1 / 49.2, 4 000 tiles 144 / 122.  A transposed,
+    // K 32: 252 tiles 12.1 / 11.3, 752 tiles 31.0 / 23.2, 1 876 tiles
+    // 53.5 / 51.5; K 64: 512 tiles 25.3 / 22.2, 1 064 tiles 41.6 / 44.3.
+    const bool gelu = g.epi == EPI_BIAS_GELU || g.epi == EPI_BIAS_GELU_D || g.epi == EPI_GELU;
+    const bool brief = g.a_t ? 16 * tiles > 11 * cu && g.K <= (tiles < 4 * cu ? 64 : 32)
+                             : tiles > 2 * cu && g.K <= (tiles <= 3 * cu || (gelu && tiles > 6 * cu) ? 48 : 16);
+    bool tail = true;   // balance a partial last wave by K splits (see pt_gemm)
+    if (brief && !bf && vec && g.dma && dma_ok(g) && !g.f32m) {
+        g.f32m = 1;
+        g.small = 0;
+        splits = 1;
+        tail = false;   // of two stages each: two more launches than they save
+    }
     if (have_ws || g.Mdev) {
         if (pt_gemm_ksplit_fits(g)) {
             g.small = 2;
             splits = 1;
         }
     }
-    return GemmPlan{vec, bf, wsplit_ok, bk, cu, tiles, tiles_s, splits};
+    return GemmPlan{vec, bf, wsplit_ok, tail, bk, cu, tiles, tiles_s, splits};
 }
 
 // ptcg_kernel_gemm_path's codes
@@ -3798,7 +3819,7 @@ int pt_gemm(const GemmArgs& g0, float* ws, long ws_floats, hipStream_t s) {
     // the time).  Run the first T - T % S tiles whole and split the tail's K
     // across the idle CUs, then reduce the tail partials in a fixed order.
     // Worth its two extra launches only while a CU holds few tiles (T < 4 S).
-    if (!db && !g.Mdev && !g.small && ws != nullptr) {
+    if (!db && !g.Mdev && !g.small && plan.tail && ws != nullptr) {
         const int S = pt_cu_count();
         const int R = S > 0 ? tiles % S : 0;
         const int ksteps = pt_cdiv(g.K, bk);

@@ -60,3 +60,16 @@ def test_long_k_is_split_over_the_chip(M, N, b_t):
     for K in (2052, 4096, 16384, 1 << 20):
         assert path(M, N, K, b_t=b_t) in (SMALL, SPLIT)
     assert path(M, N, 4096, b_t=b_t, rows_dev=1) == (KSPLIT if M < 2000 else SMALL)
+
+
+@pytest.mark.parametrize("M,N", [(65540, 128), (16400, 512), (9000, 1024)])   # 513..568 tiles on 256 CUs
+def test_short_k_on_wide_grids_runs_on_fp32_instructions(M, N):
+    """A few k stages past the split's two workgroups per CU."""
+    for a_t, b_t in ((0, 0), (0, 1), (1, 1), (1, 0)):
+        for K in (4, 16, 20, 48):
+            assert path(M, N, K, a_t=a_t, b_t=b_t) == F32
+        assert path(M, N, 68, a_t=a_t, b_t=b_t) in (SPLIT, SMALL)
+    assert path(M, N, 16, rows_dev=1) == F32
+    assert path(60000, 128, 16) == SPLIT          # 469 tiles: one round of workgroups
+    assert path(200000, 64, 48) == SPLIT          # 1 563 tiles
+    assert path(200000, 64, 48, a_t=1, b_t=1) == SPLIT and path(200000, 64, 32, a_t=1, b_t=1) == F32

@@ -58,6 +58,37 @@ def test_edges(M, N, K, a_t, b_t, cuda):
     assert rel_l2(C.cpu(), ref.cpu()) < bound(K), rel_l2(C.cpu(), ref.cpu())
 
 
+# a few k stages on wide grids: the fp32 instructions in every layout
+@pytest.mark.parametrize("a_t,b_t", [(0, 0), (0, 1), (1, 1), (1, 0)])
+@pytest.mark.parametrize("M,N,K", [(33000, 132, 4), (65540, 128, 16), (65540, 128, 20), (16396, 508, 48)])
+def test_short_k(M, N, K, a_t, b_t, cuda):
+    A, B, a, b = operands(M, N, K, a_t, b_t)
+    g = torch.Generator().manual_seed(M)
+    bias, R = torch.randn(N, generator=g).cuda(), torch.randn(M, N, generator=g).cuda()
+    C = gemm(a, b, M, N, K, a_t, b_t, 3, bias, R)
+    ref = A.cuda().double() @ B.cuda().double() + bias.double() + R.double()
+    assert rel_l2(C.cpu(), ref.cpu()) < 2.0 ** -24 * (2 + math.sqrt(K / 2))   # an addition per two k
+
+
+@pytest.mark.parametrize("rows", [4, 20, 64])
+def test_short_weight_gradient(rows, cuda):
+    """dW and its bias sums over one to four k stages, and the same over a
+    device row count."""
+    L, n_out, n_in = native.lib(), 33000, 132
+    g = torch.Generator("cuda").manual_seed(rows)
+    dY, X = (torch.randn(rows, n, device="cuda", generator=g) for n in (n_out, n_in))
+    dW, db = torch.zeros(n_out, n_in, device="cuda"), torch.zeros(n_out, device="cuda")
+    ws, nd = torch.zeros(32 << 20, device="cuda"), torch.tensor([rows - 3], dtype=torch.int32, device="cuda")
+    for n in (rows, rows - 3):
+        a = (rows, n_in, n_out, P(dY), n_out, P(X), n_in, P(dW), P(db))
+        native.check(L.ptcg_kernel_gemm_dw(*a, P(ws), ws.numel(), None) if n == rows else
+                     L.ptcg_kernel_gemm_dw_rows_dev(*a, P(nd), P(ws), ws.numel(), None))
+        torch.cuda.synchronize()
+        tol = 2.0 ** -24 * (2 + math.sqrt(rows / 2))
+        assert rel_l2(dW.cpu(), (dY[:n].double().T @ X[:n].double()).cpu()) < tol
+        assert rel_l2(db.cpu(), dY[:n].double().sum(0).cpu()) < 2.0 ** -24 * (2 + math.sqrt(rows))
+
+
 # the 64-tile kernel, and K over the waves of 32 x 32 tiles: row, column and k
 # edges, waves with no or a partial stage, more stages than are in flight
 @pytest.mark.parametrize("ws_floats", [0, 32 << 20])
