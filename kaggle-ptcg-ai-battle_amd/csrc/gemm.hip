@@ -1755,6 +1755,7 @@ __device__ __forceinline__ void resid_ln_epilogue(const GemmArgs& g, const float
         // (rows past M are computed on R's first row and not stored)
 #pragma unroll
         for (int r0 = 0; r0 < 8; r0 += 4) {
+            if (m0 + 32 * h + 8 * wave + r0 >= g.M) break;   // uniform over the wave, no barrier below
             floatx4 x[4];
             float mu[4], rs[4];
 #pragma unroll
