@@ -949,12 +949,19 @@ __device__ __forceinline__ void gemm_dma_tile(const GemmArgs& g0, int k_chunk0, 
 // An fp32 value is split exactly into three bf16 terms x = h + m + l (h and m
 // round x and x - h to nearest even, l is what is left: 8 + 8 + 8 significand
 // bits and the signs of m and l cover the 24 of x).  A product keeps the six
-// terms down to 2^-18 of it (hh, hm, mh, mm, hl, lh); the three it drops are
-// below 2^-26.  A 16-k step sums its six v_mfma_f32_32x32x16_bf16, small
-// terms first, from zero and adds the result to the fp32 accumulators once,
-// where v_mfma_f32_32x32x2_f32 rounds them eight times: the relative L2 error
-// against 64 bits is 0.9e-7 / 1.7e-7 / 3.2e-7 at K = 256 / 1 024 / 4 096 where
-// the fp32 instruction's is 2.9e-7 / 5.7e-7 / 1.15e-6 (N(0, 1) operands).
+// terms hh, hm, mh, mm, hl, lh.  Of the three it drops, m l and l m are up to
+// 2^-25 of the product each (x = y = 1 + 2^-8 - 2^-17: m = 2^-8, l = -2^-17,
+// with one sign, so nothing averages out over k) and l l 2^-34: about 2^-24 in
+// all at most.  A 16-k step is six
+// v_mfma_f32_32x32x16_bf16: hh onto one accumulator, the five small terms onto
+// another, both running over all of K and added once at the end.  The large
+// one is rounded once per 16 k, where v_mfma_f32_32x32x2_f32 rounds eight
+// times.  Relative L2 error against 64 bits, split / fp32 instruction, units
+// of 2^-24: N(0, 1) operands 1.5 / 4.8 at K = 256, 3.1 / 9.6 at 1 024, 6.7 /
+// 19.3 at 4 096; uniform on [1, 2) 0.5 / 4.0, 3.2 / 8.0, 5.8 / 16.0; all 1 +
+// 2^-8 - 2^-17, 0.99 / 0.99 at any K; and the split's worst case, operands just
+// below that at K = 4, 0.94 / 0.66 (from K = 16 0.92 / 1.04).  A sum of one
+// product may be an ulp off where the fp32 instruction's is half of one.
 // Rates measured on this GPU with random operands: 1 738 TFLOP/s for the bf16
 // instruction (its clock drops with the operands' switching), so 290 for six,
 // against 155 for the fp32 one.
@@ -1011,7 +1018,8 @@ __device__ __forceinline__ Frag3 split_frag(const float (&x)[8]) {
     return Frag3{__builtin_bit_cast(bf16x8, s.h), __builtin_bit_cast(bf16x8, s.m), __builtin_bit_cast(bf16x8, s.l)};
 }
 // hi[ti] += the hh term and lo[ti] += the five small terms of b x a[ti] over
-// a 16-k step for one 32-column slice
+// a 16-k step for one 32-column slice (in the order that keeps the two chains
+// apart)
 template <int TA>
 __device__ __forceinline__ void mma_split(floatx16 (&hi)[TA], floatx16 (&lo)[TA], const Frag3 (&a)[TA],
                                           const Frag3& b) {

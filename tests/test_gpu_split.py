@@ -2,10 +2,12 @@
 tile and k edges of the 128 x 128, 64 x 64 and 32 x 32 kernels, non-finite, extreme
 and tiny operands, operands past 2^31 bytes, and the residual + LayerNorm forms.
 
-Tolerance: a 16-k step's products are summed exactly to 2^-26 and added to the
-fp32 accumulators once, so K / 16 roundings of 2^-24 (random signs) and the
-final one: relative L2 <= 2^-24 (2 + sqrt(K / 16)) against float64.  Split-K
-partials are summed in fp32, one more rounding per split (at most K / 16).
+Tolerance, relative L2 against float64: the dropped terms m l and l m are at
+most 2^-25 of a product each, with one sign at worst (2^-24); the accumulator of
+the large terms is rounded once per 16 k (2^-24 each, random signs), the small
+terms' roundings are 2^-8 of those, and the two are added once (2^-24): 2^-24 (2
++ sqrt(K / 16)).  Split-K partials are summed in fp32, one more rounding per
+split (at most K / 16 in all, counted above).
 """
 import math
 
@@ -87,6 +89,20 @@ def test_short_weight_gradient(rows, cuda):
         tol = 2.0 ** -24 * (2 + math.sqrt(rows / 2))
         assert rel_l2(dW.cpu(), (dY[:n].double().T @ X[:n].double()).cpu()) < tol
         assert rel_l2(db.cpu(), dY[:n].double().sum(0).cpu()) < 2.0 ** -24 * (2 + math.sqrt(rows))
+
+
+@pytest.mark.parametrize("M,K", [(4, 4), (96, 4), (96, 16), (23000, 64), (512, 256), (512, 4096)])
+@pytest.mark.parametrize("spread", [0.0, 0.5])
+def test_one_sign_of_dropped_terms(M, K, spread, cuda):
+    """Operands at and just below 1 + 2^-8 - 2^-17, whose dropped terms are the
+    largest there are and all of one sign.  All roundings may share a sign too:
+    K / 16 of them, on partial sums of half the result on average."""
+    N = 128
+    g = torch.Generator().manual_seed(K)
+    A, B = (1 + 2.0 ** -8 - 2.0 ** -17 * (1 + spread * torch.rand(s, generator=g)) for s in ((M, K), (K, N)))
+    C = gemm(A, B.T, M, N, K, 0, 0)
+    ref = A.double() @ B.double()
+    assert rel_l2(C.cpu(), ref) < 2.0 ** -24 * (2 + K / 32), rel_l2(C.cpu(), ref) * 2 ** 24
 
 
 # the 64-tile kernel, and K over the waves of 32 x 32 tiles: row, column and k
