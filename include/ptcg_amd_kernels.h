@@ -51,6 +51,21 @@ int ptcg_kernel_gemm_rows_dev(int M, int N, int K, const float* A, int64_t lda, 
                               const float* R, int64_t ldr, float* C2, int64_t ldc2, const int* rows_dev,
                               float* workspace, int64_t workspace_floats, void* stream);
 
+/* The forward's products in the forms the model launches them, for parity
+ * tests at sizes of a caller's choosing: C (M, N) = epi(A B^T), A (M, K) at
+ * row stride lda, B (N, K) at row stride ldb.  form: 0 a rollout's (as
+ * ptcg_kernel_gemm), 1 a training step's (fp32 matrix instructions), 2 bf16
+ * products of fp32 operands (as ptcg_kernel_gemm_bf16), 3 bf16-stored
+ * operands (as ptcg_kernel_gemm_bs; C and C2 bf16 except for epi 3).  epi as
+ * ptcg_kernel_gemm, and 9: C = gelu(acc + bias[n]), a rollout's GELU layer.
+ * rows_dev (nullable) as ptcg_kernel_gemm_rows_dev; workspace as
+ * ptcg_kernel_gemm (not used by form 3).
+ * No reference counterpart: the launch forms of pt_linear's products.      */
+int ptcg_kernel_gemm_fwd(int form, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
+                         void* C, int64_t ldc, int epi, const float* bias, const void* R, int64_t ldr, void* C2,
+                         int64_t ldc2, const int* rows_dev, float* workspace, int64_t workspace_floats,
+                         void* stream);
+
 /* C = alpha * op(A) op(B) + beta * R (R may not alias C), the alpha / beta
  * form of cublasGemmExDense / puf_addmm_nn (native/src/kernels.cu:262-310)
  * that the reference's Muon Newton-Schulz steps use (muon.cu:270-282);
@@ -135,6 +150,11 @@ int ptcg_kernel_layernorm_fwd(const float* x, const float* w, const float* b, fl
 int ptcg_kernel_gemm_resid_ln(int rows, int K, const void* A, const void* W, const float* bias,
                               const float* R, float* C, const float* lnw, const float* lnb, void* y,
                               float* mean, float* rstd, int bf16, const int* rows_dev, void* stream);
+/* ptcg_kernel_gemm_resid_ln in fp32 as a training step's forward launches it
+ * (fp32 matrix instructions).                                             */
+int ptcg_kernel_gemm_resid_ln_train(int rows, int K, const float* A, const float* W, const float* bias,
+                                    const float* R, float* C, const float* lnw, const float* lnb, float* y,
+                                    float* mean, float* rstd, const int* rows_dev, void* stream);
 int ptcg_kernel_layernorm_bwd(const float* dy, const float* x, const float* w,
                               const float* mean, const float* rstd, const float* dres,
                               float* dx, float* dw, float* db, int rows, int D,

@@ -47,6 +47,35 @@ extern "C" int ptcg_kernel_gemm_rows_dev(int M, int N, int K, const float* A, in
     return pt_gemm(g, workspace, workspace_floats, (hipStream_t)stream);
 }
 
+extern "C" int ptcg_kernel_gemm_fwd(int form, int M, int N, int K, const void* A, int64_t lda, const void* B,
+                                    int64_t ldb, void* C, int64_t ldc, int epi, const float* bias, const void* R,
+                                    int64_t ldr, void* C2, int64_t ldc2, const int* rows_dev, float* workspace,
+                                    int64_t workspace_floats, void* stream) {
+    PT_REQUIRE(A && B && C, "kernel_gemm_fwd: null operand");
+    PT_REQUIRE(form >= 0 && form <= 3, "kernel_gemm_fwd: bad form %d", form);
+    PT_REQUIRE((epi >= EPI_STORE && epi <= EPI_MUL) || epi == EPI_GELU, "kernel_gemm_fwd: bad epilogue %d", epi);
+    PT_REQUIRE(!((epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_BIAS_RESID || epi == EPI_BIAS_GELU_D ||
+                  epi == EPI_GELU) && !bias),
+               "kernel_gemm_fwd: epilogue %d needs bias", epi);
+    PT_REQUIRE(!((epi == EPI_BIAS_RESID || epi == EPI_GELU_BWD || epi == EPI_MUL) && !R),
+               "kernel_gemm_fwd: epilogue %d needs R", epi);
+    PT_REQUIRE(!((epi == EPI_BIAS_GELU || epi == EPI_BIAS_GELU_D) && !C2), "kernel_gemm_fwd: epilogue %d needs C2",
+               epi);
+    GemmArgs g{};
+    g.M = M; g.N = N; g.K = K;
+    g.A = static_cast<const float*>(A); g.lda = lda;
+    g.B = static_cast<const float*>(B); g.ldb = ldb;
+    g.C = static_cast<float*>(C); g.ldc = ldc; g.epi = epi;
+    g.bias = bias; g.R = static_cast<const float*>(R); g.ldr = ldr;
+    g.C2 = static_cast<float*>(C2); g.ldc2 = ldc2;
+    g.Mdev = rows_dev;
+    g.f32m = form == 1;
+    g.prec = form >= 2;
+    g.bs = form == 3;
+    g.obf = form == 3 && epi != EPI_BIAS_RESID;
+    return pt_gemm(g, workspace, workspace_floats, (hipStream_t)stream);
+}
+
 extern "C" int ptcg_kernel_gemm_axpby(int M, int N, int K, const float* A, int64_t lda, int a_t,
                                       const float* B, int64_t ldb, int b_t, float* C, int64_t ldc, float alpha,
                                       const float* R, int64_t ldr, float beta, void* stream) {
@@ -179,6 +208,23 @@ extern "C" int ptcg_kernel_gemm_resid_ln(int rows, int K, const void* A, const v
     g.epi = EPI_BIAS_RESID;
     g.Mdev = rows_dev;
     return pt_gemm_resid_ln(g, lnw, lnb, static_cast<float*>(y), 256, mean, rstd, (hipStream_t)stream, bf16);
+}
+
+extern "C" int ptcg_kernel_gemm_resid_ln_train(int rows, int K, const float* A, const float* W, const float* bias,
+                                               const float* R, float* C, const float* lnw, const float* lnb,
+                                               float* y, float* mean, float* rstd, const int* rows_dev,
+                                               void* stream) {
+    PT_REQUIRE(rows > 0 && K > 0, "kernel_gemm_resid_ln_train: empty shape %d x %d", rows, K);
+    GemmArgs g{};
+    g.M = rows; g.N = 256; g.K = K;
+    g.f32m = 1;
+    g.A = A; g.lda = K;
+    g.B = W; g.ldb = K;
+    g.C = C; g.ldc = 256;
+    g.bias = bias; g.R = R; g.ldr = 256;
+    g.epi = EPI_BIAS_RESID;
+    g.Mdev = rows_dev;
+    return pt_gemm_resid_ln(g, lnw, lnb, y, 256, mean, rstd, (hipStream_t)stream, 0);
 }
 
 extern "C" int ptcg_kernel_gemm_dx_layernorm_bwd(int rows, int K, const void* dY, const void* WT, const float* x,

@@ -211,6 +211,10 @@ _SIGS = {
         ctypes.c_int, ctypes.c_int, ctypes.c_int, c_void_p, ctypes.c_int64, c_void_p, ctypes.c_int64,
         ctypes.c_int, c_void_p, ctypes.c_int64, ctypes.c_int, c_void_p, c_void_p, ctypes.c_int64, c_void_p,
         ctypes.c_int64, c_void_p, c_void_p, ctypes.c_int64, c_void_p]),
+    "ptcg_kernel_gemm_fwd": (ctypes.c_int, [
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, c_void_p, ctypes.c_int64, c_void_p, ctypes.c_int64,
+        c_void_p, ctypes.c_int64, ctypes.c_int, c_void_p, c_void_p, ctypes.c_int64, c_void_p, ctypes.c_int64,
+        c_void_p, c_void_p, ctypes.c_int64, c_void_p]),
     "ptcg_kernel_gemm_bf16": (ctypes.c_int, [
         ctypes.c_int, ctypes.c_int, ctypes.c_int, c_void_p, ctypes.c_int64, ctypes.c_int,
         c_void_p, ctypes.c_int64, ctypes.c_int, c_void_p, ctypes.c_int64, ctypes.c_int,
@@ -237,6 +241,7 @@ _SIGS = {
                                           c_void_p, c_void_p, ctypes.c_int64, c_void_p]),
     "ptcg_kernel_gemm_resid_ln": (ctypes.c_int, [ctypes.c_int, ctypes.c_int] + [c_void_p] * 10 + [ctypes.c_int]
                                   + [c_void_p] * 2),
+    "ptcg_kernel_gemm_resid_ln_train": (ctypes.c_int, [ctypes.c_int, ctypes.c_int] + [c_void_p] * 12),
     "ptcg_kernel_layernorm_fwd": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p,
                                                  c_void_p, c_void_p, ctypes.c_int, ctypes.c_int,
                                                  c_void_p]),
