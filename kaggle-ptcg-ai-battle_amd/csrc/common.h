@@ -295,7 +295,7 @@ int pt_dx_lnbwd(const GemmArgs& g, const float* x, const float* w, const float* 
 
 // One product of a grouped launch (pt_gemm_grouped): all products of a
 // launch share the operand layout (a_t, b_t) and epilogue, and must meet the
-// LDS-DMA tile rules (16 B-aligned operands, leading dimensions multiples of
+// split kernel's tile rules (16 B-aligned operands, leading dimensions multiples of
 // 4, K a multiple of 16 for k-contiguous operands).  Split-K products write
 // `splits` partials of M x ldc at g.C (part_stride apart) and
 // pt_grouped_reduce sums them into out.

@@ -1,16 +1,18 @@
-// fp32 GEMM on CDNA4 matrix cores (v_mfma_f32_16x16x4_f32), LDS-staged.
+// GEMMs on CDNA4 matrix cores: fp32 on the bf16 pipe by a three-way operand split
+// (the default), fp32 on fp32 instructions, and bf16 products.
 //
 // Replaces the reference's cuBLAS GemmEx wrappers pt_gemm / pt_linear /
-// pt_linear_bwd / pt_bias_grad (native/model/ptcg_kernels.cuh:42-108) with
-// one templated kernel: 128x128 block tile, BK = 16, 256 threads = 4 waves
-// in a 2x2 grid, each wave a 64x64 sub-tile of 4x4 MFMA 16x16 tiles.
+// pt_linear_bwd / pt_bias_grad (native/model/ptcg_kernels.cuh:42-108).
+// gemm_f32_kernel, for operands off the LDS-DMA rules: 128x128 block tile, BK =
+// 16, 256 threads = 4 waves in a 2x2 grid, each wave a 64x64 sub-tile of 4x4
+// v_mfma_f32_16x16x4_f32 tiles.
 // Global->LDS moves 128-bit vectors along whichever dimension is contiguous
 // in memory, double buffered (the prefetch of tile t+1 overlaps the MFMAs of
 // tile t), and is stored without transposition; the MFMA k order is chosen
 // so a k-contiguous fragment is a single 128-bit LDS read per four MFMA
-// steps.  Tiles are ordered per XCD (L2 reuse of the A rows).  Epilogues
-// fuse bias, exact GELU (keeping the pre-activation), residual add and the
-// GELU backward multiply.  Weight gradients (K = rows, small M*N) split K
+// steps.  In every kernel tiles are ordered per XCD (L2 reuse of the A rows) and
+// epilogues fuse bias, exact GELU (keeping the pre-activation), residual add and
+// the GELU backward multiply.  Weight gradients (K = rows, small M*N) split K
 // across blocks and sum the partials in a fixed order, so results do not
 // depend on scheduling (the reference accumulates with atomics).
 #include "common.h"
@@ -735,7 +737,7 @@ __device__ __forceinline__ void store_tile32(const GemmArgs& g, floatx16 (&acc32
 }
 
 // One 128 x 128 tile of C (split bz of gz along K) of the logical tile
-// index bx; shared by the per-product launch and the grouped launch.
+// index bx: fp32 instructions (the training forward, short K) or bf16 products.
 // NS: pipeline stages (NS - 1 tiles in flight while one is multiplied).
 // fp32 products: a wave's 64 x 64 tile is 2 x 2 tiles of
 // v_mfma_f32_32x32x2_f32 (153.6 TFLOP/s measured on this GPU against 139.6
@@ -758,20 +760,8 @@ __device__ __forceinline__ void gemm_dma_tile(const GemmArgs& g0, int k_chunk0, 
                                               int gz, float* smem) {
     constexpr bool W32 = !BF;
     const GemmArgs g = gemm_shape(g0);
-    // a device reduction count splits its own K evenly over the launch's
-    // splits, or (wsplit) as many ways as the weight-gradient rule gives for
-    // that count: the later splits return, and workgroup (0, 0, 0) leaves the
-    // count after the partials (and bias partials) for the reduce
-    int k_chunk = g0.Kdev ? (((g.K + gz - 1) / gz + BK - 1) / BK) * BK : k_chunk0;
-    if constexpr (PARTIAL) {
-        if (g0.Kdev && g0.wsplit) {
-            const int tiles = ((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
-            const int sp = pt_split_chunks(g.K, min(pt_wgrad_splits(g.K, tiles, g0.wsplit, BK), gz), BK, &k_chunk);
-            if (bx == 0 && bz == 0 && threadIdx.x == 0)
-                *reinterpret_cast<int*>(g0.C + (long)gz * (part_stride + (DB ? g0.M : 0))) = sp;
-            if (bz >= sp) return;
-        }
-    }
+    // a device reduction count splits its own K evenly over the launch's splits
+    const int k_chunk = g0.Kdev ? (((g.K + gz - 1) / gz + BK - 1) / BK) * BK : k_chunk0;
     constexpr int TILE = BM * BK;   // floats per operand tile (BM == BN)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tn = (g.N + BN - 1) / BN;
@@ -896,26 +886,17 @@ __device__ __forceinline__ void gemm_dma_tile(const GemmArgs& g0, int k_chunk0, 
                 else bf[t] = make_float4(Bb[dma_at<true>(cb, 4 * lq)], Bb[dma_at<true>(cb, 4 * lq + 1)],
                                          Bb[dma_at<true>(cb, 4 * lq + 2)], Bb[dma_at<true>(cb, 4 * lq + 3)]);
             }
-            if constexpr (BF) {
-                bf16x4 ah[4], bh[4];
+            bf16x4 ah[4], bh[4];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    ah[t] = to_bf16x4(af[t].x, af[t].y, af[t].z, af[t].w);
-                    bh[t] = to_bf16x4(bf[t].x, bf[t].y, bf[t].z, bf[t].w);
-                }
-#pragma unroll
-                for (int ti = 0; ti < 4; ++ti)
-#pragma unroll
-                    for (int tj = 0; tj < 4; ++tj)
-                        acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[tj], ah[ti], acc[ti][tj], 0, 0, 0);
-            } else {
-#define PT_MFMA_STEP(c)                                                                             \
-            _Pragma("unroll") for (int ti = 0; ti < 4; ++ti)                                        \
-            _Pragma("unroll") for (int tj = 0; tj < 4; ++tj)                                        \
-                acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[tj].c, af[ti].c, acc[ti][tj], 0, 0, 0);
-            PT_MFMA_STEP(x) PT_MFMA_STEP(y) PT_MFMA_STEP(z) PT_MFMA_STEP(w)
-#undef PT_MFMA_STEP
+            for (int t = 0; t < 4; ++t) {
+                ah[t] = to_bf16x4(af[t].x, af[t].y, af[t].z, af[t].w);
+                bh[t] = to_bf16x4(bf[t].x, bf[t].y, bf[t].z, bf[t].w);
             }
+#pragma unroll
+            for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+                for (int tj = 0; tj < 4; ++tj)
+                    acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bh[tj], ah[ti], acc[ti][tj], 0, 0, 0);
             if (do_db) {
                 // k rows past K were loaded as zeros; columns past M are never stored
 #pragma unroll
@@ -1095,14 +1076,15 @@ template <bool T> struct SplitSlot {
 // A 128 x 128 tile of C by 4 waves of 64 x 64.  Each operand element is read
 // to registers once per workgroup, split there and written to LDS as three
 // bf16 planes ([row][16 k], the two 16 B halves of a row swapped every eight
-// rows: conflict-free writes and fragment reads), two stages; splitting at the fragment reads instead (fp32 in LDS by DMA) splits every
-// element twice.  Two stages of loads are in flight where A is k-contiguous, one
-// where it is transposed (see AHEAD; one: 149 504 x 256 x 1 024 500 us, two:
-// 458; x 768 x 256 423 and 404; 8192^3 5.92 and 5.45 ms); one barrier per
-// stage.  A transposed operand (weight gradients) is read row by row of k and
-// needs no transposition: the eight k of a slot are eight registers.
-// Same split-K, device-count, tail-partial and bias-sum rules as
-// gemm_dma_tile.
+// rows: conflict-free writes and fragment reads), two stages; splitting at the
+// fragment reads instead (fp32 in LDS by DMA) splits every element twice.  Two
+// stages of loads are in flight where A is k-contiguous, one where it is
+// transposed (see AHEAD; one: 149 504 x 256 x 1 024 500 us, two: 458; x 768 x
+// 256 423 and 404; 8192^3 5.92 and 5.45 ms); one barrier per stage.  A
+// transposed operand (weight gradients) is read row by row of k and needs no
+// transposition: the eight k of a slot are eight registers.
+// Split-K, device-count, tail-partial and bias-sum rules as gemm_dma_tile's,
+// and a device reduction count may choose its own splits (wsplit).
 constexpr int SPLIT_FLOATS = 2 * 2 * 3 * BM * BK / 2;   // two stages
 static_assert(SPLIT_FLOATS >= STAGE_FLOATS, "epilogue stage does not fit the operand stages");
 __device__ __forceinline__ int split_at(int r, int kg) { return r * BK + 8 * (kg ^ ((r >> 3) & 1)); }
@@ -1113,6 +1095,10 @@ __device__ __forceinline__ void gemm_split_tile(const GemmArgs& g0, int k_chunk0
     constexpr int T = BM, TT = 2;   // tile size, 32 x 32 slices per wave side
     constexpr int PLANE = T * BK, OPER = 3 * PLANE, STAGE = 2 * OPER;   // bf16 elements
     const GemmArgs g = gemm_shape(g0);
+    // a device reduction count splits its own K evenly over the launch's
+    // splits, or (wsplit) as many ways as the weight-gradient rule gives for
+    // that count: the later splits return, and workgroup (0, 0, 0) leaves the
+    // count after the partials (and bias partials) for the reduce
     int k_chunk = g0.Kdev ? (((g.K + gz - 1) / gz + BK - 1) / BK) * BK : k_chunk0;
     if constexpr (PARTIAL) {
         if (g0.Kdev && g0.wsplit) {
@@ -1344,7 +1330,7 @@ __device__ __forceinline__ void gemm_small_tile(const GemmArgs& g0, int k_chunk0
     const GemmArgs g = gemm_shape(g0);
     int k_chunk = g0.Kdev ? (((g.K + gz - 1) / gz + BK - 1) / BK) * BK : k_chunk0;
     if constexpr (PARTIAL) {
-        if (g0.Kdev && g0.wsplit) {   // see gemm_dma_tile
+        if (g0.Kdev && g0.wsplit) {   // see gemm_split_tile
             const int tiles = ((g.M + SM_T - 1) / SM_T) * ((g.N + SM_T - 1) / SM_T);
             const int sp = pt_split_chunks(g.K, min(pt_wgrad_splits(g.K, tiles, g0.wsplit, BK), gz), BK, &k_chunk);
             if (bx == 0 && bz == 0 && threadIdx.x == 0)
@@ -1668,7 +1654,7 @@ __device__ __forceinline__ DTail dtail_plan(const GemmArgs& g, int S) {
 // would need an agent-scope release per tail workgroup (an L2 write-back on
 // this GPU, measured slower than the unbalanced wave).
 template <bool AT, bool BT, int EPI, bool SPLIT>
-__global__ __launch_bounds__(NT) void gemm_f32_dma_dtail_kernel(const GemmArgs g0, float* __restrict__ part,
+__global__ __launch_bounds__(NT) void gemm_dtail_kernel(const GemmArgs g0, float* __restrict__ part,
                                                                int S) {
     __shared__ __align__(16) float smem[SPLIT ? SPLIT_FLOATS : dma_smem_floats<DMA_NS>()];
     const DTail p = dtail_plan(gemm_shape(g0), S);
@@ -1692,7 +1678,7 @@ __global__ __launch_bounds__(NT) void gemm_f32_dma_dtail_kernel(const GemmArgs g
     else gemm_dma_tile<AT, BT, EPI, true, false>(q, p.kc, 0, u % p.R, u / p.R, p.s2, smem);
 }
 
-// The tail tiles of gemm_f32_dma_dtail_kernel: 16 workgroups per tail tile
+// The tail tiles of gemm_dtail_kernel: 16 workgroups per tail tile
 // (tile-major, so the launch's S * 16 workgroups past R * 16 return), each
 // thread one float4 of tile t: its s2 partials summed in split order through
 // the epilogue (tail_reduce_kernel's arithmetic, the plan taken from the
@@ -2225,19 +2211,19 @@ __global__ __launch_bounds__(NT) void gemm_dx_lnbwd_kernel(const GemmArgs g0, co
             ((red[c] + red[2 * RL_N + c]) + red[4 * RL_N + c]) + red[6 * RL_N + c];
 }
 
-// Grouped launch: several independent products (different shapes and
-// operands, one layout and epilogue) in one grid.  Work item w belongs to
+// Grouped launch (the Muon step's): several independent products (different
+// shapes and operands, one layout and epilogue) in one grid, on the split.  Work item w belongs to
 // product item_group[w]; its logical tile and K split follow from the
 // product's first item, tile count and split count.
 template <bool AT, bool BT, int EPI, bool PARTIAL>
-__global__ __launch_bounds__(NT) void gemm_f32_dma_grouped_kernel(const GroupedGemm* __restrict__ gs,
-                                                                  const int* __restrict__ item_group) {
+__global__ __launch_bounds__(NT) void gemm_split_grouped_kernel(const GroupedGemm* __restrict__ gs,
+                                                                const int* __restrict__ item_group) {
     __shared__ __align__(16) float smem[SPLIT_FLOATS];
     const int gi = __builtin_amdgcn_readfirstlane(item_group[blockIdx.x]);
     const int local = (int)blockIdx.x - gs[gi].first;
     const int tiles = gs[gi].tiles;
     gemm_split_tile<AT, BT, EPI, PARTIAL, false>(gs[gi].g, gs[gi].k_chunk, gs[gi].part_stride, local % tiles,
-                                                     local / tiles, gs[gi].splits, smem);
+                                                 local / tiles, gs[gi].splits, smem);
 }
 
 // Fixed-order sums of grouped split-K partials: chunk c covers 1024
@@ -3561,15 +3547,15 @@ int pt_dx_lnbwd(const GemmArgs& g, const float* x, const float* w, const float* 
                       ws_floats - (long)blocks * 2 * RL_N, s);
 }
 
-// the device-decided balanced last wave: gemm_f32_dma_dtail_kernel, then
+// the device-decided balanced last wave: gemm_dtail_kernel, then
 // dtail_reduce_kernel over its tail partials in ws
 template <bool AT, bool BT, int EPI>
 static void launch_dtail(const GemmArgs& g, int tiles, int S, float* ws, hipStream_t s) {
     const int slot = pt_prof_open(s);
     if (g.f32m)
-        hipLaunchKernelGGL((gemm_f32_dma_dtail_kernel<AT, BT, EPI, false>), dim3(tiles + S), dim3(NT), 0, s, g, ws, S);
+        hipLaunchKernelGGL((gemm_dtail_kernel<AT, BT, EPI, false>), dim3(tiles + S), dim3(NT), 0, s, g, ws, S);
     else
-        hipLaunchKernelGGL((gemm_f32_dma_dtail_kernel<AT, BT, EPI, true>), dim3(tiles + S), dim3(NT), 0, s, g, ws, S);
+        hipLaunchKernelGGL((gemm_dtail_kernel<AT, BT, EPI, true>), dim3(tiles + S), dim3(NT), 0, s, g, ws, S);
     pt_prof_close(slot, g_gemm_class, launch_flops(g), s);
     hipLaunchKernelGGL(dtail_reduce_kernel<EPI>, dim3(S * DTAIL_RED_WG), dim3(256), 0, s, g, (const float*)ws, S);
 }
@@ -3886,11 +3872,11 @@ template <bool AT, bool BT>
 int launch_grouped(const GroupedGemm* d, const int* ig, int items, int epi, int partial, hipStream_t s) {
     const dim3 grid(items), blk(NT);
     if (partial && epi == EPI_STORE)
-        hipLaunchKernelGGL((gemm_f32_dma_grouped_kernel<AT, BT, EPI_STORE, true>), grid, blk, 0, s, d, ig);
+        hipLaunchKernelGGL((gemm_split_grouped_kernel<AT, BT, EPI_STORE, true>), grid, blk, 0, s, d, ig);
     else if (!partial && epi == EPI_STORE)
-        hipLaunchKernelGGL((gemm_f32_dma_grouped_kernel<AT, BT, EPI_STORE, false>), grid, blk, 0, s, d, ig);
+        hipLaunchKernelGGL((gemm_split_grouped_kernel<AT, BT, EPI_STORE, false>), grid, blk, 0, s, d, ig);
     else if (!partial && epi == EPI_AXPBY)
-        hipLaunchKernelGGL((gemm_f32_dma_grouped_kernel<AT, BT, EPI_AXPBY, false>), grid, blk, 0, s, d, ig);
+        hipLaunchKernelGGL((gemm_split_grouped_kernel<AT, BT, EPI_AXPBY, false>), grid, blk, 0, s, d, ig);
     else
         PT_REQUIRE(false, "gemm_grouped: epilogue %d (partial %d) not supported", epi, partial);
     PT_LAUNCH_CHECK();

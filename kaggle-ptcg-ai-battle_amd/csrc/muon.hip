@@ -20,10 +20,11 @@
 // is M x N with M <= N, zero-padded to multiples of 16; per-matrix
 // normalisation), one launch applies every matrix update, and each
 // Newton-Schulz phase is ONE grouped GEMM launch over all matrices' tiles
-// (the LDS-DMA MFMA kernel; the Gram products split K and a grouped
-// fixed-order reduce sums them; the alpha / beta epilogue forms b A + c A A
-// and a X + B X).  The padding keeps every product on the DMA tile rules and
-// stays exactly zero through the iteration.  A step is ~30 launches where
+// (fp32 on the bf16 matrix pipe by the three-way split, gemm.hip; the Gram
+// products split K and a grouped fixed-order reduce sums them; the alpha /
+// beta epilogue forms b A + c A A and a X + B X).  The padding keeps every
+// product on the split's tile rules and stays exactly zero through the
+// iteration.  A step is ~30 launches where
 // the reference issues ~20 per matrix; the grads are read, never written
 // (the reference clips and transforms them in place).
 #include "model.h"
