@@ -155,11 +155,6 @@ template <class Op> __device__ __forceinline__ float wave_reduce(float v, Op op)
 __device__ __forceinline__ float wave_sum(float v) {
     return wave_reduce(v, [](float a, float b) { return a + b; });
 }
-// the sum of a product, its first step a fused multiply-add: own product
-// unrounded, the other half's rounded
-__device__ __forceinline__ float wave_sum_prod(float a, float b) {
-    return half_reduce(__builtin_fmaf(a, b, __shfl_xor(a * b, 32, 64)), [](float x, float y) { return x + y; });
-}
 __device__ __forceinline__ float wave_max(float v) {
     return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }

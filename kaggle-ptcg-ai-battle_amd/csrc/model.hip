@@ -170,6 +170,10 @@ struct PtcgModel {
 // the next step by up to 2e-5 of the output's norm (3 of 23 seeds above 1e-5
 // after one step), where the backward's moves it by up to
 // 2e-6 (32 seeds).
+// So a rollout's log-probabilities and the same weights' in the first epoch of
+// training come from two arithmetics, and the first minibatch's ratios differ
+// from 1 by the rounding of both (outputs within about 1e-6 of 64 bits in
+// either, relative L2), not by that of tile plans alone.
 //
 // A GELU layer's forward keeps gelu'(z) for the backward (EPI_BIAS_GELU_D: Y
 // = gelu', Y2 = gelu); a rollout has none, so its layers write gelu(z) alone
@@ -222,9 +226,10 @@ struct LnOut {
 // 119 vs ~133, K 1024: 231 vs ~213.  In the CORE step (FFN2 at K 1024
 // unfused) +0.4% replayed, +0.8% stream-launched; the reference variant's
 // FFN2 at K 512 x 82.4k rows (280 vs ~258 alone) ran 0.3% slower unfused in
-// its step, so it stays fused.  Both give the same bits.  Few rows of a rollout
-// run apart as well, where the product takes 32 x 32 tiles with K over a
-// workgroup's waves (1 168 rows at K 256: 16.7 us fused, 6.3 + 4.7 apart).
+// its step, so it stays fused.  Without K splits both give the same bits.  Few
+// rows of a rollout run apart as well, where the product takes 32 x 32 tiles
+// with K over a workgroup's waves, which sums K in eight parts (1 168 rows at K
+// 256: 16.7 us fused, 6.3 + 4.7 apart).
 static int lin_resid_ln(const PtcgModel* m, const float* X, const float* W, const float* b, float* Y, int rows,
                         int in, int out, const float* R, const LnOut& ln, hipStream_t s, const int* Mdev) {
     GemmArgs g{};
@@ -716,7 +721,7 @@ static size_t carve(PtcgModel* m, char* base) {
     m->bw.resize(d.layers);
     for (auto& w : m->bw) carve_bw(c, w, d);
     if (crit) carve_bw(c, m->cbw, d);
-    if (!train) {   // forward GEMMs use the workspace for balanced tail tiles only
+    if (!train) {   // forward GEMMs: balanced tail tiles and K splits
         m->ws_floats = 4L << 20;
         m->ws = c.take(m->ws_floats);
         return c.off;

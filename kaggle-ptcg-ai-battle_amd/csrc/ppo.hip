@@ -43,6 +43,16 @@ __device__ __forceinline__ float block_sum4(float v, float* red, int tid) {
     return ((red[0] + red[1]) + red[2]) + red[3];
 }
 
+// sum of a b over the wave, its first step a fused multiply-add: own product
+// unrounded, that of lane ^ 32 rounded.  Which one is rounded differs between
+// the lane halves and no later step crosses them, so lanes 0-31 and 32-63 hold
+// sums that may differ in rounding (each the row's entropy to fp32).  The form
+// is kept for its bits: the rounding of this sum reaches the optimizer through
+// score_mlp.2.bias, whose gradient is otherwise 0 (see model.hip).
+__device__ __forceinline__ float entropy_sum(float a, float b) {
+    return half_reduce(__builtin_fmaf(a, b, __shfl_xor(a * b, 32, 64)), [](float x, float y) { return x + y; });
+}
+
 __global__ __launch_bounds__(256) void ppo_loss_kernel(PPOArgs a) {
     __shared__ float red[4];
     __shared__ float rowstat[4][NSTAT];
@@ -107,9 +117,7 @@ __global__ __launch_bounds__(256) void ppo_loss_kernel(PPOArgs a) {
         const float lse = mx + logf(sum);
         const float logp = on ? l[j] - lse : 0.f;
         const float p = on ? expf(logp) : 0.f;
-        // (the rounding of this sum reaches the optimizer through
-        // score_mlp.2.bias, whose gradient is otherwise 0: see model.hip)
-        const float ent = -wave_sum_prod(p, logp);
+        const float ent = -entropy_sum(p, logp);
         const float lp_act = __shfl(logp, act[j], 64);
         const float adv_n = (adv[j] - mean) / (adv_std + 1e-8f);
         // value loss + gradient (pufferlib.cu:1068-1085)
