@@ -48,6 +48,11 @@ sys.path.insert(0, ROOT)
 METRIC = "PPO minibatch step obs/sec (fwd+bwd+Adam) @B=512; % MFMA/HBM roofline"
 FP32_MFMA_PEAK_TFLOPS = 157.3      # MI355X dense fp32 matrix peak
 BF16_MFMA_PEAK_TFLOPS = 2500.0     # MI355X dense bf16 matrix peak
+# fp32 products on the bf16 pipe by a three-way operand split: six bf16 products each
+SPLIT_MFMA_PEAK_TFLOPS = BF16_MFMA_PEAK_TFLOPS / 6
+# an fp32 training step: the forward's third of the useful flops on fp32
+# instructions, the backward's two thirds on the split, each at its pipe's peak
+FP32_STEP_PEAK_TFLOPS = 1 / (1 / 3 / FP32_MFMA_PEAK_TFLOPS + 2 / 3 / SPLIT_MFMA_PEAK_TFLOPS)
 HBM_PEAK_GBS = 8000.0              # MI355X HBM3E bandwidth
 # launch classes of ptcg_profile_class: (index, name); amounts are HBM bytes
 HBM_CLASSES = ((1, "layernorm_fwd"), (2, "layernorm_bwd"), (3, "adam_norm"), (4, "adam_update"),
@@ -441,11 +446,12 @@ def main():
         lv.append(l)
     gemm_s = ms.value / 1e3
     achieved = useful / gemm_s / 1e12
-    peak = BF16_MFMA_PEAK_TFLOPS if bf16 else FP32_MFMA_PEAK_TFLOPS
+    peak = BF16_MFMA_PEAK_TFLOPS if bf16 else round(FP32_STEP_PEAK_TFLOPS, 1)
     traffic = measured_gemm_traffic()
     kname = ("gemm_bs32_kernel + gemm_bs_dw_kernel + gemm_resid_ln_kernel + gemm_dx_lnbwd_kernel (trunk blocks, "
              "bf16 operands) + gemm_bf16_k16_kernel"
-             if bf16 else "gemm_f32_dma_kernel + gemm_f32_kernel + gemm_resid_ln_kernel")
+             if bf16 else "gemm_split_kernel (backward) + gemm_f32_dma_kernel + gemm_resid_ln_kernel (forward) + "
+             "gemm_small_kernel + gemm_ksplit_kernel + gemm_f32_kernel")
     roof = dict(bound="mfma", kernel=f"{kname} (all launches: trunk, token, option and head GEMMs)",
                 achieved=round(achieved, 3), peak=peak, unit="TFLOP/s",
                 frac=round(achieved / peak, 4),
@@ -457,6 +463,9 @@ def main():
                 executed_tflops=round(exec_flops.value / gemm_s / 1e12, 3),
                 useful_tflop_per_step=round(useful / K / 1e12, 4),
                 mean_valid_seq=round(float(np.mean(lv)), 2))
+    if not bf16:
+        roof["peak_note"] = (f"forward products on fp32 matrix instructions ({FP32_MFMA_PEAK_TFLOPS} TFLOP/s), backward "
+                             f"products as six bf16 ones ({SPLIT_MFMA_PEAK_TFLOPS:.1f}), weighted by their flops")
     if not bf16 and dm.d == 256:
         roof["fused_layernorm"] = ("the blocks' residual products (out-projection, FFN2) run the LayerNorm that "
                                    "reads their output in the same launch (gemm_resid_ln_kernel): its time and "
@@ -572,6 +581,7 @@ def bench_rollout(args):
     useful_fwd = useful / 3.0
     gemm_s = ms.value / 1e3
     achieved = useful_fwd * K / gemm_s / 1e12
+    peak = BF16_MFMA_PEAK_TFLOPS if bf else SPLIT_MFMA_PEAK_TFLOPS
     line = {
         "metric": "rollout forward + action sampling obs/sec @8192 rows" + (", bf16 products" if bf else ""),
         "value": round(n * K / sec, 2),
@@ -584,10 +594,11 @@ def bench_rollout(args):
                    "sampler": args.sampler,
                    "rows": n, "seq_len": dm.l_tok + 1, "parallelism": "single GPU",
                    "launch": "HIP graph replay (step captured once)" if graph else "stream"},
-        "roofline": dict(bound="mfma", kernel=("gemm_bf16_k16_kernel" if bf else "gemm_f32_dma_kernel + gemm_f32_kernel")
-                         + " (forward GEMMs)", achieved=round(achieved, 3),
-                         peak=BF16_MFMA_PEAK_TFLOPS if bf else FP32_MFMA_PEAK_TFLOPS, unit="TFLOP/s",
-                         frac=round(achieved / (BF16_MFMA_PEAK_TFLOPS if bf else FP32_MFMA_PEAK_TFLOPS), 4),
+        "roofline": dict(bound="mfma", kernel=("gemm_bs32_kernel + gemm_resid_ln_kernel + gemm_bf16_k16_kernel" if bf else
+                                               "gemm_split_kernel + gemm_split_resid_ln_kernel + gemm_ksplit_kernel + "
+                                               "gemm_f32_dma_kernel + gemm_f32_kernel")
+                         + " (forward GEMMs)", achieved=round(achieved, 3), peak=round(peak, 1), unit="TFLOP/s",
+                         frac=round(achieved / peak, 4),
                          traffic=None, gemm_ms_per_step=round(ms.value / K, 4),
                          launches_per_step=launches.value / K, mean_valid_seq=round(lv, 2)),
     }
