@@ -3666,7 +3666,8 @@ static GemmPlan gemm_plan(GemmArgs& g, bool have_ws) {
     // tiles 27 / 29, 94 tiles 36 / 42, and over a device row count (no
     // splits) 104 tiles 62 / 39, 160 tiles 63 / 42, 314 tiles 64 / 80; weight
     // gradients of 3 000 rows, 4 tiles 24 / 14, 12 tiles 25 / 22, 16 tiles
-    // 25 / 25; of 10 000 rows, 4 tiles 24 / 23, 12 tiles 38 / 56.
+    // 25 / 25; of 10 000 rows, 4 tiles 24 / 23, 12 tiles 38 / 56.  (The bounds
+    // are this GPU's, of 256 CUs, as are pt_gemm_ksplit_fits's.)
     if (!bf && vec && g.dma && dma_ok(g)) {
         if (g.f32m) {
             // the training forward keeps its splits: they are part of its rounding

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(MC_T) void mlp_chain_fwd_kernel(const MlpChain a) {
     mc_dense<MC_R>(gdl, bin, bin, a.bcw, a.bcb, a.D, false, a.bc, a.D, nullptr, 0, nullptr, 0, row0, nrows);
 }
 
-// Up to one workgroup per CU of one sample each: forward at 16 samples 39.8 ->
+// Up to one workgroup per CU (256) of one sample each: forward at 16 samples 39.8 ->
 // 20.6 us, backward at 40 samples 65 -> 49 us; the whole step or rollout gains
 // up to 256 samples (step of 256: 4 766 -> 4 733 us).  The sums do not depend
 // on R.
